@@ -131,8 +131,10 @@ int pe_gemm(const pe_gemm_desc* d, const void* a, const void* b, float* c, void*
 /* The tile and K split pe_gemm takes for these extents and strides, operand
  * pointers taken as 16-byte aligned (no counterpart in the reference; for
  * tests and tuning): info[0..3] = tile rows, tile columns, K splits, k per
- * split (256 x 256 for the large float16 kernel).  The split, and so the
- * workspace size, is the same for every operand layout. */
+ * split (256 x 256 for the large float16 kernel; 1, 1 for a matrix-vector
+ * product, M or N = 1 and the other operand contiguous along k or its free
+ * axis).  But for matrix-vector products, the split, and so the workspace
+ * size, is the same for every operand layout; it never depends on addresses. */
 int pe_gemm_choice(const pe_gemm_desc* d, int64_t* info);
 
 /* Fused linear-attention chain.  No single entry point of the reference

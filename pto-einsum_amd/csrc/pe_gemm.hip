@@ -2,6 +2,7 @@
 // classification, tile / split-K choice and the deterministic split-K
 // reduction kernel.
 #include "pe_gemm_kernel.h"
+#include "pe_gemv.h"
 
 #include <algorithm>
 
@@ -620,6 +621,16 @@ extern "C" int pe_gemm_choice(const pe_gemm_desc* d, int64_t* info) {
     if (!d || !info) return pe::fail(PE_ERR_INVALID, "gemm_choice: null argument");
     const int st = pe::validate_gemm(*d);
     if (st != PE_OK) return st;
+    const int64_t nb = pe::batch_total(*d);
+    if (nb > 0 && d->K > 0) {
+        const pe::GemvPlan v = pe::gemv_plan(*d, nb);
+        if (v.kind) {
+            info[0] = info[1] = 1;
+            info[2] = v.split;
+            info[3] = v.kps;
+            return PE_OK;
+        }
+    }
     // As pe_gemm chooses for these strides, operand pointers taken as
     // 16-byte aligned (the split is the same for every layout).
     const int vec = d->dtype == PE_F32 ? 4 : 8;
@@ -650,7 +661,8 @@ extern "C" int pe_gemm_choice(const pe_gemm_desc* d, int64_t* info) {
 extern "C" int64_t pe_gemm_workspace_bytes(const pe_gemm_desc* d) {
     if (!d || pe::validate_gemm(*d) != PE_OK) return 0;
     if (d->K == 0 || d->M == 0 || d->N == 0 || pe::batch_total(*d) == 0) return 0;
-    return pe::choose(*d).ws_bytes;
+    const pe::GemvPlan v = pe::gemv_plan(*d, pe::batch_total(*d));
+    return v.kind ? v.ws_bytes : pe::choose(*d).ws_bytes;
 }
 
 extern "C" int pe_gemm(const pe_gemm_desc* d, const void* a, const void* b, float* c, void* ws,
@@ -680,6 +692,19 @@ extern "C" int pe_gemm(const pe_gemm_desc* d, const void* a, const void* b, floa
         r.nsplit = 0;
         r.partial = nullptr;
         PE_CHECK_HIP(launch_splitk_reduce(r, s));
+        return PE_OK;
+    }
+
+    const GemvPlan v = gemv_plan(*d, nb);
+    if (v.kind) {  // a matrix-vector product
+        if (v.ws_bytes > 0 && (!ws || ws_bytes < v.ws_bytes))
+            return fail(PE_ERR_WORKSPACE, "gemm: split-K workspace missing or too small");
+        PE_CHECK_HIP(launch_gemv(*d, v, nb, a, b, c, ws, s));
+        if (v.split > 1 && v.split <= kWaveReduceSplits) {
+            r.nsplit = v.split;
+            r.partial = static_cast<const float*>(ws);
+            PE_CHECK_HIP(launch_splitk_reduce(r, s));
+        }
         return PE_OK;
     }
 
