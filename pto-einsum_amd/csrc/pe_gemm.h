@@ -133,6 +133,10 @@ hipError_t launch_gemm_res(int dtype, int alayout, int blayout, const GemmArgs& 
 // for other dtypes, layouts and tiles).
 int gemm_ks_resident(int dtype, int alayout, int blayout, int tile);
 hipError_t launch_gemm_ks(int dtype, int alayout, int blayout, int tile, const GemmArgs& g, hipStream_t s);
+// Register-staged 16-bit MFMA kernel (pe_gemm_rs.h): 64x64 or 128x128 tiles
+// (`tile`), float16 operands or float32 ones as three bfloat16 terms, L_MN or
+// L_K at any alignment, output strides as gemm_dl_eligible asks.
+hipError_t launch_gemm_rs(int dtype, int tile, int alayout, int blayout, const GemmArgs& g, hipStream_t s);
 // Large float16 kernel (pe_gemm_big.h): 256x256 tiles, one block per CU,
 // operands L_MN or L_K under the gemm_dl_eligible conditions, no K split.
 // gemm_big_resident: resident blocks per CU (0 when it spilled).

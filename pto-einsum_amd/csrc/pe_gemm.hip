@@ -74,6 +74,27 @@
 // = 2) is not chosen automatically: on the GDN 16x16 contractions (256 x
 // 128^3, one 128x128 tile per CU) it took 20.8-22.6 us against 18.9-19.6 us
 // for 64x64 tiles of the two-stage kernel at four blocks per CU.
+// float32 GEMMs of at least this K take the register-staged kernel's 128x128
+// tiles (three bfloat16 terms per element, two blocks per CU) when those give
+// seven tenths of the CUs one, or the K split of choose() gives every CU 1.8.
+// Measured on one MI355X against the float32 MFMA kernels: 16 x 1024 x 1536,
+// K = 128 62.8 -> 53.9 us, 192 83.8 -> 72.4, 256 107.9 -> 88.9, 512 208.8 ->
+// 154.0; 2048^3 153 -> 114, 4096^3 984 -> 740, 8192 x 2048 x 2048 520 -> 380,
+// 4096 x 128 x 4096 (16 splits) 48.7 -> 43.0, 2304^2 x 6144 (7) 538 -> 403;
+// one tile per CU: 2048^2 x 512 40.9 -> 34.5, 16 x 512^3 43.0 -> 35.1, half a
+// CU's: 2048^2 x 256 (64x64 tiles before) 24.4 -> 22.8.  Shorter K is bound by
+// loads and stores, which two blocks per CU keep fewer of in flight than the
+// direct-load kernel's four (the GDN products, 1024 x 128^3, 52.2 -> 56.4).
+#ifndef PE_GEMM_RS_F32_MIN_K
+#define PE_GEMM_RS_F32_MIN_K 192
+#endif
+// ... and operands that the direct-load kernel cannot take (unaligned rows or
+// bases; element loads otherwise) from this K: 2001 x 3003, K = 75 21.9 ->
+// 17.3 us, 131 31.0 -> 23.7 and (k contiguous) 33.8 -> 22.5.
+#ifndef PE_GEMM_RS_F32_MIN_K_ANY
+#define PE_GEMM_RS_F32_MIN_K_ANY 64
+#endif
+
 #ifndef PE_GEMM_RES
 #define PE_GEMM_RES 1
 #endif
@@ -515,6 +536,12 @@ bool dl_off32(const pe_gemm_desc& d) {
     return span_ok(d.a_ms, d.a_ks) && span_ok(d.b_ns, d.b_ks);
 }
 
+// The register-staged kernel's: (128 rows, 64 k) of both operands.
+bool rs_off32(const pe_gemm_desc& d) {
+    const int64_t elem = d.dtype == PE_F32 ? 4 : 2, lim = int64_t(1) << 32;
+    return (128 * d.a_ms + 64 * d.a_ks) * elem < lim && (128 * d.b_ns + 64 * d.b_ks) * elem < lim;
+}
+
 // float16 products with K in (96, 128] (four 32-k slabs) that the tile
 // choice leaves unsplit on 128x128 tiles, at most
 // PE_GEMM_RES_MAX_TILES_PER_CU of those per CU: the short-K kernel, all of K
@@ -553,6 +580,67 @@ hipError_t launch_res(const pe_gemm_desc& d, const void* a, const void* b, float
         g.c_bs[i] = d.c_bstride[i];
     }
     return launch_gemm_res(d.dtype, al, bl, g, s);
+}
+
+// Layout of an operand for the register-staged kernel (pe_gemm_rs.h), at any
+// alignment: L_MN or L_K where that axis is contiguous and at least a vector
+// long, else L_GENERIC.
+int rs_layout(int64_t rows, int64_t k, int64_t rs, int64_t ks, int vec) {
+    if (rows >= vec && rs == 1) return L_MN;
+    if (k >= vec && ks == 1) return L_K;
+    return L_GENERIC;
+}
+
+// Whether the register-staged kernel takes d (by extents and strides, never
+// by addresses), and the operands' layouts for it.
+bool rs_eligible(const pe_gemm_desc& d, int& al, int& bl) {
+    const int vec = d.dtype == PE_F32 ? 4 : 8;
+    al = rs_layout(d.M, d.K, d.a_ms, d.a_ks, vec);
+    bl = rs_layout(d.N, d.K, d.b_ns, d.b_ks, vec);
+    const int64_t lim = int64_t(1) << 29;  // 32-bit store offsets, as gemm_dl_eligible
+    return d.tile == 0 && d.split_k == 0 && al != L_GENERIC && bl != L_GENERIC &&
+           255 * (d.c_ms + d.c_ns) < lim && 255 * (d.N + 1) < lim;
+}
+
+// The register-staged kernel's tile and K split for d, if it is the one to
+// run: float16 operands that the direct-load kernels cannot take (dl false),
+// float32 ones by PE_GEMM_RS_F32_MIN_K's rule.
+bool rs_choice(const pe_gemm_desc& d, bool dl, int& al, int& bl, GemmChoice& ch) {
+    if ((d.dtype == PE_F16 && dl) || !rs_eligible(d, al, bl)) return false;
+    ch = choose(d);
+    if (d.dtype == PE_F16) {
+        // A handful of 128x128 tiles: 64x64 ones (300 x 200 x 100 16.7 -> 6.8
+        // us; from one tile in eight CUs the larger win, 501 x 537 x 503 15.3
+        // against 19.8).
+        if (16 * ch.nbatch_total * ceil_div(d.M, 128) * ceil_div(d.N, 128) * ch.nsplit <= cu_count())
+            ch.bm = ch.bn = 64;
+        // Splits in whole 64-k slabs (no more of them, so the workspace of
+        // choose() holds).
+        if (ch.nsplit > 1) {
+            ch.k_per_split = int(ceil_div(ch.k_per_split, 64) * 64);
+            ch.nsplit = int(ceil_div(d.K, ch.k_per_split));
+        }
+        return true;
+    }
+    if (d.K < (dl ? PE_GEMM_RS_F32_MIN_K : PE_GEMM_RS_F32_MIN_K_ANY) || d.M <= 64 || d.N <= 64) return false;
+    const int64_t tiles = ch.nbatch_total * ceil_div(d.M, 128) * ceil_div(d.N, 128), cus = cu_count();
+    const bool whole = 10 * tiles >= 7 * cus;
+    const bool split = ch.bm == 128 && ch.nsplit > 1 && 10 * tiles * ch.nsplit >= 18 * cus;
+    // Busiest CU's k, at 0.74 of the rate for a CU with one block (2048^2 x
+    // 512, one tile per CU, 34.5 us; two per CU 51), plus the split's second
+    // launch and partials.
+    auto cost = [&](int64_t n, int64_t kps) {
+        const int64_t per = ceil_div(tiles * n, cus);
+        return double(per) * double(kps) / (per == 1 ? 0.74 : 1.0) +
+               (n > 1 ? 100.0 + 3.2e-5 * double(n) * double(ch.nbatch_total) * double(d.M) * double(d.N) : 0.0);
+    };
+    if (split && (!whole || cost(ch.nsplit, ch.k_per_split) < cost(1, d.K))) return true;
+    if (!whole) return false;
+    ch.bm = ch.bn = 128;
+    ch.nsplit = 1;
+    ch.k_per_split = int(d.K);
+    ch.ws_bytes = 0;
+    return true;
 }
 
 int classify(int64_t rows, int64_t k, int64_t rs, int64_t ks, const int64_t* bs, int nb,
@@ -643,7 +731,15 @@ extern "C" int pe_gemm_choice(const pe_gemm_desc* d, int64_t* info) {
         info[3] = d->K;
         return PE_OK;
     }
-    const pe::GemmChoice c = pe::choose(*d, dl, al, bl);
+    int ral, rbl;
+    pe::GemmChoice c{};
+    if (pe::rs_choice(*d, dl, ral, rbl, c)) {
+        info[0] = info[1] = c.bm;
+        info[2] = c.nsplit;
+        info[3] = c.k_per_split;
+        return PE_OK;
+    }
+    c = pe::choose(*d, dl, al, bl);
     if (d->tile == 2 || pe::res_auto(*d, c, dl, al, bl)) {
         info[0] = pe::gemm_res_tile_m(d->dtype);
         info[1] = pe::gemm_res_tile_n(d->dtype);
@@ -662,7 +758,13 @@ extern "C" int64_t pe_gemm_workspace_bytes(const pe_gemm_desc* d) {
     if (!d || pe::validate_gemm(*d) != PE_OK) return 0;
     if (d->K == 0 || d->M == 0 || d->N == 0 || pe::batch_total(*d) == 0) return 0;
     const pe::GemvPlan v = pe::gemv_plan(*d, pe::batch_total(*d));
-    return v.kind ? v.ws_bytes : pe::choose(*d).ws_bytes;
+    if (v.kind) return v.ws_bytes;
+    // (float32: the register-staged kernel's own split; its choice for
+    // float16 depends on the addresses and stays within choose()'s.)
+    int al, bl;
+    pe::GemmChoice c{};
+    if (d->dtype == PE_F32 && pe::rs_choice(*d, true, al, bl, c)) return c.ws_bytes;
+    return pe::choose(*d).ws_bytes;
 }
 
 extern "C" int pe_gemm(const pe_gemm_desc* d, const void* a, const void* b, float* c, void* ws,
@@ -746,8 +848,11 @@ extern "C" int pe_gemm(const pe_gemm_desc* d, const void* a, const void* b, floa
         PE_CHECK_HIP(launch_res(*d, a, b, c, nb, al, bl, s));
         return PE_OK;
     }
-    GemmChoice ch = choose(*d, dl, al, bl);
-    if (dl && gemm_dl_resident(d->dtype, ch.bm, ch.bn, ch.minb, al, bl) < 1) {
+    int ral, rbl;
+    GemmChoice ch{};
+    const bool rs = rs_choice(*d, dl, ral, rbl, ch);
+    if (!rs) ch = choose(*d, dl, al, bl);
+    if (!rs && dl && gemm_dl_resident(d->dtype, ch.bm, ch.bn, ch.minb, al, bl) < 1) {
         // the chosen direct-load instantiation spills: the staged kernel
         dl = false;
         ch = choose(*d, false, al, bl);
@@ -783,7 +888,7 @@ extern "C" int pe_gemm(const pe_gemm_desc* d, const void* a, const void* b, floa
     // 4096 22.6 against 26.4, 1664 x 2304 x 3072 with 3.7 tiles per CU 48.8
     // against 60.1).
     const int64_t cus = cu_count();
-    if (res_auto(*d, ch, dl, al, bl)) {
+    if (!rs && res_auto(*d, ch, dl, al, bl)) {
         PE_CHECK_HIP(launch_res(*d, a, b, c, nb, al, bl, s));
         return PE_OK;
     }
@@ -801,7 +906,7 @@ extern "C" int pe_gemm(const pe_gemm_desc* d, const void* a, const void* b, floa
         ks_k = ch.nsplit > 1 && tiles64 <= 3 * cus &&
                ((tiles64 >= cus && d->K <= 8 * PE_GEMM_KS_MAX_K) || (4 * tiles64 >= cus && d->K <= 2 * PE_GEMM_KS_MAX_K));
     }
-    if (ks_k && dl && d->split_k == 0 && d->tile == 0 && gemm_ks_resident(d->dtype, al, bl, ks_tile) >= 1) {
+    if (ks_k && dl && !rs && d->split_k == 0 && d->tile == 0 && gemm_ks_resident(d->dtype, al, bl, ks_tile) >= 1) {
         GemmArgs g{};
         g.a = a; g.b = b; g.c = c;
         g.partial = nullptr;
@@ -849,8 +954,9 @@ extern "C" int pe_gemm(const pe_gemm_desc* d, const void* a, const void* b, floa
         g.b_bs[i] = d->b_bstride[i];
         g.c_bs[i] = d->c_bstride[i];
     }
-    g.off32 = dl && dl_off32(*d);
-    hipError_t e = dl                   ? launch_gemm_dl(d->dtype, ch.bm, ch.bn, ch.minb, al, bl, !hbm_bound(*d), g, s)
+    g.off32 = rs ? rs_off32(*d) : dl && dl_off32(*d);
+    hipError_t e = rs                   ? launch_gemm_rs(d->dtype, ch.bm, ral, rbl, g, s)
+                   : dl                   ? launch_gemm_dl(d->dtype, ch.bm, ch.bn, ch.minb, al, bl, !hbm_bound(*d), g, s)
                    : d->dtype == PE_F32 ? launch_gemm_f32(ch.bm, ch.bn, al, bl, ch.persist, g, s)
                                         : launch_gemm_f16(ch.bm, ch.bn, al, bl, PE_GEMM_F16_PERSIST, g, s);
     PE_CHECK_HIP(e);

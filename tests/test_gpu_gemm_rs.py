@@ -1,0 +1,108 @@
+"""Register-staged GEMM (pe_gemm_rs.h): float16 operands that are not whole
+aligned vectors and float32 operands as three bfloat16 terms, at the edges of
+tiles, vectors and slabs, in every operand layout, against float64."""
+import ctypes
+
+import pytest
+import torch
+
+from pto_einsum import abi, einsum, launch
+
+pytestmark = pytest.mark.gpu
+
+EPS = 2.0 ** -24
+LAYOUTS = ["bij,bjk->bik", "bij,bkj->bik", "bji,bjk->bik", "bji,bkj->bik"]
+
+
+def _operands(eq, nb, M, N, K, dtype, seed, off=0):
+    d = dict(b=nb, i=M, j=K, k=N)
+    g = torch.Generator().manual_seed(seed)
+    out = []
+    for s in eq.split("->")[0].split(","):
+        shape = [d[c] for c in s]
+        n = shape[0] * shape[1] * shape[2]
+        out.append(torch.randn(n + off, generator=g).to(dtype).cuda()[off:].view(shape))
+    return out
+
+
+def _check(eq, a, b, K):
+    """Within K roundings of sum |a||b|, the bound of any order of K fused
+    terms (the split's omitted part is below half a rounding per term), each
+    2^-24 of a normal result or 2^-150 of a subnormal one, and the same bits
+    on a second call."""
+    got = einsum(eq, a, b)
+    want = torch.einsum(eq, a.double(), b.double())
+    mag = torch.einsum(eq, a.double().abs(), b.double().abs())
+    bad = (got.double() - want).abs() > K * (EPS * mag + 2.0 ** -150)
+    assert not bool(bad.any()), (eq, tuple(a.shape), tuple(b.shape), int(bad.sum()))
+    assert torch.equal(got, einsum(eq, a, b))
+
+
+@pytest.mark.parametrize("eq", LAYOUTS)
+@pytest.mark.parametrize("nb,M,N,K", [
+    (1, 9, 8, 9), (1, 63, 65, 8), (2, 65, 63, 15), (1, 64, 70, 33), (3, 70, 90, 31),       # 64x64 tiles, 32-k slabs
+    (20, 201, 99, 65), (1, 300, 200, 64), (1, 700, 129, 71), (40, 129, 131, 127),          # 128x128, 64-k slabs
+    (40, 136, 250, 129), (1, 1100, 1300, 193), (1, 1001, 301, 2003),                       # splits
+    (2, 2001, 1003, 1000),
+])
+def test_float16_unaligned_rows(eq, nb, M, N, K):
+    a, b = _operands(eq, nb, M, N, K, torch.float16, M + N + K)
+    _check(eq, a, b, K)
+
+
+@pytest.mark.parametrize("eq", LAYOUTS)
+@pytest.mark.parametrize("nb,M,N,K,off", [
+    (48, 129, 131, 64, 1), (48, 130, 140, 65, 0), (48, 255, 100, 79, 0), (48, 129, 257, 81, 0), (50, 200, 136, 191, 3),
+    (48, 128, 256, 192, 0), (48, 132, 252, 193, 0), (47, 133, 255, 207, 2), (1, 1700, 1800, 777, 0),
+    (1, 768, 768, 4096, 0), (1, 767, 765, 4099, 0),    # K splits
+])
+def test_float32_as_bfloat16_terms(eq, nb, M, N, K, off):
+    a, b = _operands(eq, nb, M, N, K, torch.float32, M + N + K, off)
+    _check(eq, a, b, K)
+
+
+@pytest.mark.parametrize("eq,layout", [(LAYOUTS[0], (0, 1)), (LAYOUTS[1], (0, 0)), (LAYOUTS[2], (1, 1))])
+@pytest.mark.parametrize("nb,M,N,K", [(64, 128, 384, 192), (16, 512, 512, 512), (1, 2048, 1536, 2048)])
+def test_float32_error_is_no_larger_than_float32_mfmas(eq, layout, nb, M, N, K):
+    """Against 64 bits, next to the same product on float32 matrix cores (the
+    explicit 128x128 tile)."""
+    a, b = _operands(eq, nb, M, N, K, torch.float32, 11)
+    want = torch.einsum(eq, a.double(), b.double())
+    got = einsum(eq, a, b)
+    d = launch.GemmDesc(dtype=launch.DT_F32, batch_shape=[nb], a_bstride=[M * K], b_bstride=[K * N], c_bstride=[M * N],
+                        M=M, N=N, K=K, a_ms=1 if layout[0] else K, a_ks=M if layout[0] else 1,
+                        b_ks=N if layout[1] else 1, b_ns=1 if layout[1] else K, c_ms=N, c_ns=1,
+                        a_numel=nb * M * K, b_numel=nb * K * N, c_numel=nb * M * N, split_k=1, tile=128)
+    ref = torch.empty_like(got)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert abi.bind().pe_gemm(ctypes.byref(abi.gemm_desc(d)), *(ctypes.c_void_p(t.data_ptr()) for t in (a, b, ref)),
+                              None, ctypes.c_int64(0), st) == 0
+    e = [float((x.double() - want).norm() / want.norm()) for x in (got, ref)]
+    assert e[0] <= e[1], e
+
+
+def test_float32_range():
+    """Elements and sums outside the split's range: inf and NaN reach exactly
+    the outputs whose sums hold them, tiny and subnormal elements keep their
+    float32 accuracy, sums near the largest float32 stay finite."""
+    eq, nb, M, N, K = LAYOUTS[0], 48, 130, 260, 200
+    a, b = _operands(eq, nb, M, N, K, torch.float32, 5)
+    a[3, 7, 11], b[9, 100, 20], a[20, 129, 199] = float("inf"), float("nan"), float("-inf")
+    a[30, 5] = 2.0 ** 120
+    b[30, :, 6] = 2.0 ** 9     # overflows to inf as float32 does
+    got, want = einsum(eq, a, b), torch.einsum(eq, a.double(), b.double())
+    big = want.abs() > 3.4028235677973366e38    # halfway past the largest float32
+    for f in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(f(got) & ~big, f(want) & ~big)
+    assert torch.equal(torch.isinf(got)[big], torch.ones_like(got[big], dtype=torch.bool))
+    for scale in (2.0 ** -104, 2.0 ** -126, 2.0 ** -140):
+        a, b = _operands(eq, nb, M, N, K, torch.float32, 6)
+        a[5] *= scale            # one batch wholly tiny, one element of another
+        a[7, 64, 3] *= scale
+        b[8, 5:50] *= scale
+        _check(eq, a, b, K)
+    a, b = _operands(eq, nb, M, N, K, torch.float32, 7)
+    a[4], b[4] = 2.0 ** 60, 1.9 * 2.0 ** 66 / K     # sums just below 2^127
+    a[6], b[6] = 2.0 ** 60, 1.95 * 2.0 ** 67 / K    # ... and above it
+    assert bool(torch.isfinite(einsum(eq, a, b)).all())
+    _check(eq, a, b, K)
