@@ -430,6 +430,86 @@ __global__ __launch_bounds__(kThreads) void product_rows_kernel(ProductArgs p, u
     }
 }
 
+// Products with an operand that is contiguous along another output axis (q)
+// than the innermost one (p), as in st,ts->ts: 64 x 64 tiles, that operand
+// read along q into LDS and multiplied and stored along p.  AQ: the first
+// operand runs along q too, so the product is formed on the way into LDS.
+// One element per lane and access (256 bytes a wave); LDS rows are one
+// element longer than the tile, so both its accesses are conflict-free.
+// Before, every lane fetched its own line of that operand: one MI355X, f32
+// st,ts->ts 4096^2 468 -> 40 us (5.0 TB/s), f16 433 -> 38.4, 8001 x 8003 1591
+// -> 231 (rows off the line grid), 1001 x 1003 31.6 -> 6.5; st,st->ts 471 -> 41.
+constexpr int kPT = 64;
+
+struct ProductTileArgs {
+    const void* a;
+    const void* b;
+    float* out;
+    uint32_t P, Q;          // extents along p and q
+    uint32_t tiles_p, tiles;  // tiles along p; per batch
+    int64_t a_p, a_q, b_p, o_q;  // strides (b's along q and the output's along p are 1)
+    int32_t nbatch;
+    FastDiv batch_div[kMaxOuter];
+    int64_t a_batch[kMaxOuter], b_batch[kMaxOuter], o_batch[kMaxOuter];
+    int32_t nt;
+};
+
+template <typename E, bool AQ, bool ADD_ZERO>
+__global__ __launch_bounds__(kThreads) void product_tile_kernel(ProductTileArgs g) {
+    using T = typename E::T;
+    __shared__ float tile[kPT][kPT + 1];
+    const uint32_t batch = blockIdx.x / g.tiles;
+    const uint32_t t = blockIdx.x - batch * g.tiles;
+    const uint32_t tq = t / g.tiles_p, tp = t - tq * g.tiles_p;
+    int64_t ao = 0, bo = 0, oo = 0;
+    uint32_t rem = batch;
+    for (int d = g.nbatch - 1; d >= 0; --d) {
+        uint32_t q, r;
+        g.batch_div[d].divmod(rem, q, r);
+        ao += int64_t(r) * g.a_batch[d];
+        bo += int64_t(r) * g.b_batch[d];
+        oo += int64_t(r) * g.o_batch[d];
+        rem = q;
+    }
+    const T* __restrict__ a = static_cast<const T*>(g.a) + ao;
+    const T* __restrict__ b = static_cast<const T*>(g.b) + bo;
+    float* __restrict__ out = g.out + oo;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t p0 = tp * kPT, q0 = tq * kPT;
+    const uint32_t np = min(uint32_t(kPT), g.P - p0), nq = min(uint32_t(kPT), g.Q - q0);
+    // Rows and columns past the end repeat the last ones (never stored).
+    const int64_t ql = q0 + min(lane, nq - 1);
+    float x[kPT / 4];
+#pragma unroll
+    for (int i = 0; i < kPT / 4; ++i) {
+        const int64_t p = p0 + min(uint32_t(i) * 4 + wave, np - 1);
+        x[i] = E::to_f32(b[p * g.b_p + ql]);
+    }
+    float y[kPT / 4];
+    const int64_t pl = p0 + min(lane, np - 1);
+#pragma unroll
+    for (int i = 0; i < kPT / 4; ++i) {
+        if constexpr (AQ) {
+            const int64_t p = p0 + min(uint32_t(i) * 4 + wave, np - 1);
+            y[i] = E::to_f32(a[p * g.a_p + ql]);
+        } else {
+            const int64_t q = q0 + min(uint32_t(i) * 4 + wave, nq - 1);
+            y[i] = E::to_f32(a[q * g.a_q + pl * g.a_p]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kPT / 4; ++i) tile[i * 4 + wave][lane] = AQ ? y[i] * x[i] : x[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kPT / 4; ++i) {
+        const uint32_t q = uint32_t(i) * 4 + wave;
+        const float v = tile[lane][q];
+        const float prod = AQ ? v : y[i] * v;
+        if (q < nq && lane < np)
+            store_f(out + int64_t(q0 + q) * g.o_q + p0 + lane, ADD_ZERO ? 0.0f + prod : prod, g.nt);
+    }
+}
+
 // Fallback for outputs of 2^31 elements or more: 64-bit division per element.
 template <typename E, bool ADD_ZERO>
 __global__ __launch_bounds__(kThreads) void product_kernel_wide(
@@ -500,6 +580,65 @@ hipError_t launch_rows(const ProductArgs& args, uint32_t n, bool add_zero, hipSt
     else
         hipLaunchKernelGGL((product_rows_kernel<E, AM, BM, false>), grid, dim3(kThreads), 0, s, args, n);
     return hipGetLastError();
+}
+
+// Launches product_tile_kernel if the second operand (or, swapped, the first)
+// runs along an outer axis of at least 8, as the output's inner axis is;
+// false: not such a product.
+template <typename E>
+bool launch_tiles(const ProductArgs& args, const std::vector<int64_t>& shape, bool add_zero, hipStream_t s,
+                  hipError_t& e) {
+    const int no = args.nouter;
+    const int64_t P = args.inner;
+    auto along = [&](const int64_t* outer, int64_t inner) {  // the outer axis an operand is contiguous along
+        if (inner <= 1) return -1;
+        for (int k = 0; k < no; ++k)
+            if (outer[k] == 1 && shape[k] >= 8) return k;
+        return -1;
+    };
+    int q = along(args.b_outer, args.b_inner);
+    const bool swap = q < 0;
+    if (swap) q = along(args.a_outer, args.a_inner);
+    if (q < 0 || P < 8) return false;
+    ProductTileArgs g{};
+    g.a = swap ? args.b : args.a;
+    g.b = swap ? args.a : args.b;
+    const int64_t* a_outer = swap ? args.b_outer : args.a_outer;
+    const int64_t* b_outer = swap ? args.a_outer : args.b_outer;
+    g.out = args.out;
+    g.P = uint32_t(P);
+    g.Q = uint32_t(shape[q]);
+    g.tiles_p = uint32_t(ceil_div(P, kPT));
+    g.a_p = swap ? args.b_inner : args.a_inner;
+    g.b_p = swap ? args.a_inner : args.b_inner;
+    g.a_q = a_outer[q];
+    int64_t os[kMaxOuter], st = P, batches = 1;
+    for (int k = no - 1; k >= 0; --k) {
+        os[k] = st;
+        st *= shape[k];
+    }
+    g.o_q = os[q];
+    for (int k = 0; k < no; ++k) {
+        if (k == q) continue;
+        g.batch_div[g.nbatch].init(uint32_t(shape[k]));
+        g.a_batch[g.nbatch] = a_outer[k];
+        g.b_batch[g.nbatch] = b_outer[k];
+        g.o_batch[g.nbatch] = os[k];
+        batches *= shape[k];
+        ++g.nbatch;
+    }
+    const int64_t tiles = int64_t(g.tiles_p) * ceil_div(shape[q], kPT);
+    if (tiles * batches >= (int64_t(1) << 31)) return false;
+    g.tiles = uint32_t(tiles);
+    g.nt = args.nt;
+    const bool aq = g.a_p > 1 && g.a_q == 1;
+    const dim3 grid(uint32_t(tiles * batches));
+    if (aq && add_zero) hipLaunchKernelGGL((product_tile_kernel<E, true, true>), grid, dim3(kThreads), 0, s, g);
+    else if (aq) hipLaunchKernelGGL((product_tile_kernel<E, true, false>), grid, dim3(kThreads), 0, s, g);
+    else if (add_zero) hipLaunchKernelGGL((product_tile_kernel<E, false, true>), grid, dim3(kThreads), 0, s, g);
+    else hipLaunchKernelGGL((product_tile_kernel<E, false, false>), grid, dim3(kThreads), 0, s, g);
+    e = hipGetLastError();
+    return true;
 }
 
 template <typename E>
@@ -577,7 +716,7 @@ int run(const pe_product_desc& d, const void* in0, const void* in1, float* out,
         vec_ok = (sa[k] % VEC == 0) && (args.b_inner == 0 || sb[k] % VEC == 0);
     const bool has_outer = args.nouter > 0;
 
-    hipError_t e;
+    hipError_t e = hipSuccess;
     if (vec_ok) {
         args.nvec = uint32_t(n / VEC);
         args.inner_vecs.init(uint32_t(inner / VEC));
@@ -615,7 +754,7 @@ int run(const pe_product_desc& d, const void* in0, const void* in1, float* out,
         else
             e = args.b_inner == 1 ? launch_rows<E, PM_ROW, PM_ROW>(args, un, add_zero, s)
                                   : launch_rows<E, PM_ROW, PM_ONE>(args, un, add_zero, s);
-    } else {
+    } else if (!launch_tiles<E>(args, shape, add_zero, s, e)) {
         args.nvec = uint32_t(n);
         args.inner_vecs.init(uint32_t(inner));
         if (add_zero)

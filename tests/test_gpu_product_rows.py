@@ -1,6 +1,8 @@
 """Products whose rows are not whole vectors (product_rows_kernel in
-pe_product.hip): vectors that cross rows, short rows, odd totals, unaligned
-bases and operand orders, bit-exact against torch on the CPU."""
+pe_product.hip) and products with an operand that runs along another axis than
+the output's inner one (product_tile_kernel): vectors that cross rows, short
+rows, odd totals, partial tiles, unaligned bases and operand orders, bit-exact
+against torch on the CPU."""
 import ctypes
 
 import pytest
@@ -27,6 +29,13 @@ CASES = [
     ((6, 40, 33), (33, 198, 1), (0, 33, 1)),                # A with permuted outer axes
     ((6, 40, 33), (33, 198, 1), (40, 1, 0)),                # ... times a scalar per row
     ((5, 30, 31), (930, 31, 1), (930, 31, 1)),              # merges into one axis
+    ((70, 90), (90, 1), (1, 70)),                           # tiles: B transposed
+    ((64, 64), (1, 64), (64, 1)),                           # A transposed
+    ((130, 65), (1, 130), (1, 130)),                        # both: one axis order, two of them
+    ((3, 70, 90), (6300, 90, 1), (1, 3, 210)),              # B contiguous along a short outer axis: one by one
+    ((9, 70, 90), (6300, 90, 1), (1, 9, 630)),              # ... along the first axis
+    ((5, 70, 4, 90), (25200, 360, 90, 1), (25200, 1, 6300, 70)),
+    ((70, 90), (1, 0), (1, 70)),                            # A broadcast along the row
     ((70, 3000, 37), (111000, 37, 1), (0, 0, 1)),           # 30 000 blocks
 ]
 
