@@ -607,6 +607,9 @@ bool rs_eligible(const pe_gemm_desc& d, int& al, int& bl) {
 // float32 ones by PE_GEMM_RS_F32_MIN_K's rule.
 bool rs_choice(const pe_gemm_desc& d, bool dl, int& al, int& bl, GemmChoice& ch) {
     if ((d.dtype == PE_F16 && dl) || !rs_eligible(d, al, bl)) return false;
+    if (d.dtype == PE_F32 &&
+        (d.K < (dl ? PE_GEMM_RS_F32_MIN_K : PE_GEMM_RS_F32_MIN_K_ANY) || d.M <= 64 || d.N <= 64))
+        return false;
     ch = choose(d);
     if (d.dtype == PE_F16) {
         // A handful of 128x128 tiles: 64x64 ones (300 x 200 x 100 16.7 -> 6.8
@@ -622,7 +625,6 @@ bool rs_choice(const pe_gemm_desc& d, bool dl, int& al, int& bl, GemmChoice& ch)
         }
         return true;
     }
-    if (d.K < (dl ? PE_GEMM_RS_F32_MIN_K : PE_GEMM_RS_F32_MIN_K_ANY) || d.M <= 64 || d.N <= 64) return false;
     const int64_t tiles = ch.nbatch_total * ceil_div(d.M, 128) * ceil_div(d.N, 128), cus = cu_count();
     const bool whole = 10 * tiles >= 7 * cus;
     const bool split = ch.bm == 128 && ch.nsplit > 1 && 10 * tiles * ch.nsplit >= 18 * cus;

@@ -108,8 +108,10 @@ extern "C" int pe_einsum_exec(const pe_einsum_plan* p, const void* in0, const vo
     if (p->route != PE_ROUTE_GEMM) return fail(PE_ERR_INVALID, "exec: unknown route");
     char* w = static_cast<char*>(ws);
     const bool staged = p->gather0 || p->gather1 || p->scatter_out;
-    const int64_t gws = pe_gemm_workspace_bytes(&p->gemm);
-    if ((staged || gws > 0) && !w) return fail(PE_ERR_WORKSPACE, "exec: plan needs a workspace");
+    // A workspace holds what pe_einsum_workspace_bytes asked for (this call
+    // has no size to check it by); only without one is the need worked out.
+    if (!w && (staged || pe_gemm_workspace_bytes(&p->gemm) > 0))
+        return fail(PE_ERR_WORKSPACE, "exec: plan needs a workspace");
     const void* a = in0;
     const void* b = in1;
     int st;
@@ -124,7 +126,7 @@ extern "C" int pe_einsum_exec(const pe_einsum_plan* p, const void* in0, const vo
         b = w + p->ws1_off;
     }
     float* c = p->scatter_out ? reinterpret_cast<float*>(w + p->wsout_off) : out;
-    st = run_b ? pe_gemm(&p->gemm, a, b, c, w ? w + gemm_ws_offset(*p) : nullptr, gws, stream) : PE_OK;
+    st = run_b ? pe_gemm(&p->gemm, a, b, c, w ? w + gemm_ws_offset(*p) : nullptr, w ? INT64_MAX : 0, stream) : PE_OK;
     if (st != PE_OK) return st;
     if (p->scatter_out && run_c) {
         st = pe_permute(&p->perm_out, c, out, stream);

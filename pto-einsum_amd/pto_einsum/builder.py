@@ -182,19 +182,50 @@ class EinsumBuilder:
 
             self._ws_bytes = int(abi.bind().pe_einsum_workspace_bytes(ctypes.byref(abi.einsum_plan(self.launch_plan))))
 
+        # The call's constants, and the C entry with plain pointers (the
+        # library object's own attribute keeps the reference's argtypes).
+        shape0, shape1 = (tuple(s) for s in self.input_shapes)
+        dtype, out_shape, swap = self.dtype, tuple(self.recipe["out_shape"]), self._swap_operands
+        if gpu:
+            exec_fn = self.lib["run_einsum_exec"]
+            exec_fn.argtypes, exec_fn.restype = [ctypes.c_void_p] * 5, ctypes.c_int
+
+        def launch_on(idx, inp0, inp1):
+            """Output allocation and launch with GPU ``idx`` current."""
+            if self.lib is None:
+                raise AttributeError("runner called after its builder's cleanup()")
+            dev = inp0.device
+            out = torch.empty(out_shape, dtype=torch.float32, device=dev)
+            stream = runtime.raw_stream(idx)
+            # Workspace (split-K partials, staged operands): a torch
+            # allocation per device, so creating it is stream-ordered and
+            # allowed under graph capture, and dropping it needs no
+            # synchronisation.  A use on another stream than the one it was
+            # allocated on is recorded, so the allocator does not reuse the
+            # memory before that stream's work is done.
+            entry = self._workspaces.get(idx)
+            if entry is None:
+                entry = (torch.empty(self._ws_bytes, dtype=torch.uint8, device=dev), stream)
+                self._workspaces[idx] = entry
+            elif entry[1] != stream:
+                entry[0].record_stream(torch.cuda.current_stream(dev))
+            rc = exec_fn(inp0.data_ptr(), inp1.data_ptr(), out.data_ptr(), entry[0].data_ptr(), stream)
+            if rc:
+                runtime.check(rc, "run_einsum_exec")
+            return out
+
         def run(*operands):
             if len(operands) != 2:
                 raise ValueError("Expected exactly two operands.")
             inp0, inp1 = operands
-            if tuple(inp0.shape) != tuple(self.input_shapes[0]) or \
-                    tuple(inp1.shape) != tuple(self.input_shapes[1]):
+            if inp0.shape != shape0 or inp1.shape != shape1:
                 raise ValueError(
                     f"Input shapes {inp0.shape} and {inp1.shape} do not match built shapes {self.input_shapes}.")
-            if inp0.dtype != self.dtype or inp1.dtype != self.dtype:
+            if inp0.dtype != dtype or inp1.dtype != dtype:
                 raise TypeError(
                     f"Input datatypes {inp0.dtype} and {inp1.dtype} do not match built datatype {self.dtype}.")
             if gpu:
-                if inp0.device.type != "cuda" or inp1.device != inp0.device:
+                if not inp0.is_cuda or inp1.device != inp0.device:
                     raise ValueError(
                         f"Operands must both live on one GPU for device '{self.device}', "
                         f"got {inp0.device} and {inp1.device}.")
@@ -204,36 +235,20 @@ class EinsumBuilder:
                 inp0 = inp0.contiguous()
             if not inp1.is_contiguous():
                 inp1 = inp1.contiguous()
-            if self._swap_operands:
+            if swap:
                 inp0, inp1 = inp1, inp0
-            out_shape = self.recipe["out_shape"]
             if not gpu:
                 out = torch.zeros(out_shape, dtype=torch.float32, device="cpu")
                 self.lib.run_einsum(self._ptr(inp0, self.c_type), self._ptr(inp1, self.c_type),
                                     self._ptr(out, ctypes.c_float), None)
                 return out
-            dev = inp0.device
-            with torch.cuda.device(dev):
-                out = torch.empty(out_shape, dtype=torch.float32, device=dev)
-                stream = runtime.current_stream_ptr(dev)
-                idx = dev.index if dev.index is not None else torch.cuda.current_device()
-                # Workspace (split-K partials, staged operands): a torch
-                # allocation per device, so creating it is stream-ordered and
-                # allowed under graph capture, and dropping it needs no
-                # synchronisation.  A use on another stream than the one it
-                # was allocated on is recorded, so the allocator does not
-                # reuse the memory before that stream's work is done.
-                entry = self._workspaces.get(idx)
-                if entry is None:
-                    entry = (torch.empty(self._ws_bytes, dtype=torch.uint8, device=dev), stream)
-                    self._workspaces[idx] = entry
-                elif entry[1] != stream:
-                    entry[0].record_stream(torch.cuda.current_stream(dev))
-                rc = self.lib.run_einsum_exec(self._ptr(inp0, self.c_type), self._ptr(inp1, self.c_type),
-                                              self._ptr(out, ctypes.c_float), ctypes.c_void_p(entry[0].data_ptr()),
-                                              stream)
-                runtime.check(rc, "run_einsum_exec")
-            return out
+            idx = inp0.get_device()
+            # (Entering the device context costs more than asking whether it
+            # is current already.)
+            if idx == torch.cuda.current_device():
+                return launch_on(idx, inp0, inp1)
+            with torch.cuda.device(idx):
+                return launch_on(idx, inp0, inp1)
 
         return run
 
@@ -316,27 +331,33 @@ def einsum(equation: str, *operands, device: str = "cuda", reduce_solo_axes: boo
         raise ValueError("Operands must have the same datatype.")
     if reduce_solo_axes:
         equation, inp0, inp1 = _reduce_solo_axes(equation, inp0, inp1)
-    key = (equation, tuple(inp0.shape), tuple(inp1.shape), inp0.dtype, _normalise_device(device),
+    route = "cuda" if device == "cuda" else _normalise_device(device)
+    key = (equation, inp0.shape, inp1.shape, inp0.dtype, route,
            os.getenv("EINSUM_BUILD_DIR", ""), os.getenv("EINSUM_EXTRA_DEFINES", ""))
     with _runners_lock:
         entry = _runners.get(key)
         if entry is not None:
-            _runners.move_to_end(key)
+            _use_runner(key, entry)
     if entry is None:
         builder = EinsumBuilder(equation, [inp0.shape, inp1.shape], inp0.dtype, device=device)
         entry = (builder, builder.build())
         with _runners_lock:
             _runners[key] = entry
-    with _runners_lock:
-        # No eviction while a graph is being captured: a runner used earlier
-        # in the capture must keep its workspace, which the graph reads at
-        # every replay.  The cache shrinks back at the first call after it.
-        if len(_runners) > _RUNNER_CACHE_SIZE and not _capturing():
-            while len(_runners) > _RUNNER_CACHE_SIZE:
-                _runners.popitem(last=False)
-        if _capture_pins is not None:
-            _capture_pins.append(entry)
+            _use_runner(key, entry)
     return entry[1](inp0, inp1)
+
+
+def _use_runner(key, entry) -> None:
+    """Cache upkeep of a call that uses ``entry`` (the lock is held)."""
+    _runners.move_to_end(key)
+    # No eviction while a graph is being captured: a runner used earlier in
+    # the capture must keep its workspace, which the graph reads at every
+    # replay.  The cache shrinks back at the first call after it.
+    if len(_runners) > _RUNNER_CACHE_SIZE and not _capturing():
+        while len(_runners) > _RUNNER_CACHE_SIZE:
+            _runners.popitem(last=False)
+    if _capture_pins is not None:
+        _capture_pins.append(entry)
 
 
 def _capturing() -> bool:

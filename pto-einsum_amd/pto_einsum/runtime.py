@@ -84,6 +84,15 @@ def check(status: int, what: str) -> None:
         raise RuntimeError(f"{what} failed with status {status}: {last_error()}")
 
 
+def raw_stream(index: int) -> int:
+    """The current stream's handle on GPU ``index``, without a Stream object
+    where torch offers that (0.1 against 2 us)."""
+    import torch
+
+    get = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return get(index) if get is not None else torch.cuda.current_stream(index).cuda_stream
+
+
 def current_stream_ptr(device) -> int:
     import torch
 
