@@ -2,7 +2,7 @@
 // vecmat, dot products, batched rows against rows, and the scores and values
 // of one decoded token against a key / value cache.
 //
-//   out[b, n] = sum_k W[b, n, k] * x[b, k]        (float32 fma, fixed order)
+//   out[b, n] = sum_k W[b, n, k] * x[b, k]        (fixed order, no less exact than the tiles)
 //
 // What bounds these is reading W once; the MFMA GEMMs leave 63 of 64 rows of
 // a tile idle and walk K in slabs with a barrier each.  Two kernels, by the
@@ -26,13 +26,16 @@
 //
 // Measured on one MI355X (W rotated over 1 GiB), GEMM kernels before -> now:
 // f32 8192 x 4096 matvec 46.7 -> 23.1 us (5.8 TB/s; a copy reaches 6.5), the
-// f16 scores and values of 512 heads x 2048 positions x 128 together 152 -> 93
+// f16 scores and values of 512 heads x 2048 positions x 128 together 165 -> 92
 // us.  Against these shapes: W through ordinary loads 24-31 and 50 + 55 us;
 // four rows per lane for long rows (x shared) 30 us, two 23.6; U = 2 or 8 24.4;
-// eight k in flight per thread for the columns 49, sixteen 60 us (four: 46).
+// eight k in flight per thread for the columns 49, sixteen 60 us (four: 46);
+// 64-bit lane sums exchanged through LDS instead of DPP 66 us for the scores
+// (46), pairwise sums within a lane's vector 55-58 (96 registers either way).
 #include "pe_gemv.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace pe {
 
@@ -68,12 +71,62 @@ __device__ __forceinline__ typename Vec16<E>::type ldw(const typename E::T* p) {
     else return __builtin_nontemporal_load(reinterpret_cast<const typename Vec16<E>::type*>(p));
 }
 
-// acc + sum of w[e] * x[e] in element order, one rounding per term.
+// Sum of four products as two sums of two: for float16 the first product
+// of each is exact, so a chain of four roundings at the size of the running sum
+// becomes two at a pair's, one at the four's and one at the sum's.
 template <typename E>
-__device__ __forceinline__ float dot16(typename Vec16<E>::type w, typename Vec16<E>::type x, float acc) {
+__device__ __forceinline__ float dot4(const typename E::T (&w)[4], const typename E::T (&x)[4]) {
+    const float lo = __builtin_fmaf(E::to_f32(w[1]), E::to_f32(x[1]), E::to_f32(w[0]) * E::to_f32(x[0]));
+    const float hi = __builtin_fmaf(E::to_f32(w[3]), E::to_f32(x[3]), E::to_f32(w[2]) * E::to_f32(x[2]));
+    return lo + hi;
+}
+
+// acc + w x, one rounding (in 64 bits float16's product is exact in 32).
+template <typename E, typename A>
+__device__ __forceinline__ A mad(typename E::T w, typename E::T x, A acc) {
+    if constexpr (sizeof(A) == 8) return acc + A(E::to_f32(w) * E::to_f32(x));
+    else return __builtin_fmaf(E::to_f32(w), E::to_f32(x), acc);
+}
+
+// acc + sum of w[e] * x[e] in element order.
+template <typename E, typename A>
+__device__ __forceinline__ A dot16(typename Vec16<E>::type w, typename Vec16<E>::type x, A acc) {
 #pragma unroll
-    for (int e = 0; e < Vec16<E>::V; ++e) acc = __builtin_fmaf(E::to_f32(w[e]), E::to_f32(x[e]), acc);
+    for (int e = 0; e < Vec16<E>::V; ++e) acc = mad<E, A>(w[e], x[e], acc);
     return acc;
+}
+
+// Type in which the lanes' (and the column kernel's thread rows') partial sums
+// meet: float16 operands in 64 bits, one rounding for all of them.  The matrix
+// cores round a block of products once, which chains and meets in 32 bits do
+// not reach (relative error over K = 64: tiles 5.7e-8, 32 bits 6.6e-8, this
+// 5.2e-8; the times are the same).
+template <typename E>
+struct Meet {
+    using T = float;
+};
+template <>
+struct Meet<F16> {
+    using T = double;
+};
+
+// Lane l ^ m's value (m a power of two, known when unrolled): within rows of 16
+// lanes by DPP moves, which need no LDS round trip each.
+__device__ __forceinline__ int xor_lane(int v, int m) {
+    if (m == 1) return __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xf, 0xf, false);       // quad_perm 1,0,3,2
+    if (m == 2) return __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, false);       // quad_perm 2,3,0,1
+    if (m == 4) {
+        v = __builtin_amdgcn_update_dpp(v, v, 0x141, 0xf, 0xf, false);                 // half-row mirror: ^ 7
+        return __builtin_amdgcn_update_dpp(v, v, 0x1B, 0xf, 0xf, false);               // quad_perm 3,2,1,0: ^ 3
+    }
+    if (m == 8) return __builtin_amdgcn_update_dpp(v, v, 0x128, 0xf, 0xf, false);      // row_ror 8
+    return __shfl_xor(v, m);
+}
+__device__ __forceinline__ float xor_lane(float v, int m) {
+    return __int_as_float(xor_lane(__float_as_int(v), m));
+}
+__device__ __forceinline__ double xor_lane(double v, int m) {
+    return __hiloint2double(xor_lane(__double2hiint(v), m), xor_lane(__double2loint(v), m));
 }
 
 // Offsets of batch `b` in W, x and the output.
@@ -138,11 +191,14 @@ __global__ __launch_bounds__(kThreads) void gemv_row_kernel(GemvArgs g) {
         }
     }
 
-    float acc[R][U];
+    // Rows of four vectors: all in 64 bits (K = 32: 4.4e-8 through the tiles,
+    // 5.3e-8 with a 32-bit chain).
+    using A = std::conditional_t<LPR == 4, typename Meet<E>::T, float>;
+    A acc[R][U];
 #pragma unroll
     for (int i = 0; i < R; ++i)
 #pragma unroll
-        for (int u = 0; u < U; ++u) acc[i][u] = 0.0f;
+        for (int u = 0; u < U; ++u) acc[i][u] = 0;
 
     const int nv = klen / V;
     int v0 = 0;
@@ -159,7 +215,7 @@ __global__ __launch_bounds__(kThreads) void gemv_row_kernel(GemvArgs g) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int i = 0; i < R; ++i) acc[i][u] = dot16<E>(w[i][u], x[XROW ? i : 0][u], acc[i][u]);
+            for (int i = 0; i < R; ++i) acc[i][u] = dot16<E, A>(w[i][u], x[XROW ? i : 0][u], acc[i][u]);
     }
     for (; v0 < nv; v0 += LPR) {
         if (v0 + l < nv) {
@@ -170,15 +226,16 @@ __global__ __launch_bounds__(kThreads) void gemv_row_kernel(GemvArgs g) {
 #pragma unroll
             for (int i = 0; i < (XROW ? R : 1); ++i) x[i] = ld16<E, UNAL>(xp[i] + k);
 #pragma unroll
-            for (int i = 0; i < R; ++i) acc[i][0] = dot16<E>(w[i], x[XROW ? i : 0], acc[i][0]);
+            for (int i = 0; i < R; ++i) acc[i][0] = dot16<E, A>(w[i], x[XROW ? i : 0], acc[i][0]);
         }
     }
     for (int k = nv * V + l; k < klen; k += LPR)
 #pragma unroll
         for (int i = 0; i < R; ++i)
-            acc[i][0] = __builtin_fmaf(E::to_f32(wp[i][k]), E::to_f32(xp[XROW ? i : 0][k]), acc[i][0]);
+            acc[i][0] = mad<E, A>(wp[i][k], xp[XROW ? i : 0][k], acc[i][0]);
 
-    float s[R];
+    using M = typename Meet<E>::T;
+    M s[R];
 #pragma unroll
     for (int i = 0; i < R; ++i) {
         s[i] = acc[i][0];
@@ -194,14 +251,15 @@ __global__ __launch_bounds__(kThreads) void gemv_row_kernel(GemvArgs g) {
         const bool up = (l & m) != 0;
 #pragma unroll
         for (int i = 0; i < half; ++i) {
-            const float keep = up ? s[i + half] : s[i];
-            const float send = up ? s[i] : s[i + half];
-            s[i] = keep + __shfl_xor(send, m);
+            const M keep = up ? s[i + half] : s[i];
+            const M send = up ? s[i] : s[i + half];
+            s[i] = keep + xor_lane(send, m);
         }
         held += up ? half : 0;
     }
     constexpr int kLeft = R > LPR ? R / LPR : 1;  // rows a lane still holds
-    for (; m >= 1; m /= 2) s[0] = s[0] + __shfl_xor(s[0], m);
+#pragma unroll
+    for (; m >= 1; m /= 2) s[0] = s[0] + xor_lane(s[0], m);
     // Lanes that hold the same rows: the first stores.
     constexpr int kDup = LPR > R ? LPR / R : 1;
     if (l % kDup != 0) return;
@@ -210,15 +268,15 @@ __global__ __launch_bounds__(kThreads) void gemv_row_kernel(GemvArgs g) {
         const uint32_t r = row0 + uint32_t(held + i) * G + grp;
         if (r >= nrows) continue;
         if (g.nsplit > 1) {
-            g.partial[int64_t(blockIdx.y) * g.rows + (XROW ? r : batch * uint32_t(g.N) + r)] = s[i];
+            g.partial[int64_t(blockIdx.y) * g.rows + (XROW ? r : batch * uint32_t(g.N) + r)] = float(s[i]);
         } else if constexpr (XROW) {
             uint32_t b, n;
             g.n_div.divmod(r, b, n);
             int64_t wo, xo, o;
             batch_offsets(g, b, wo, xo, o);
-            g.out[o + int64_t(n) * g.o_ns] = s[i];
+            g.out[o + int64_t(n) * g.o_ns] = float(s[i]);
         } else {
-            g.out[oo + int64_t(r) * g.o_ns] = s[i];
+            g.out[oo + int64_t(r) * g.o_ns] = float(s[i]);
         }
     }
 }
@@ -257,10 +315,15 @@ __global__ __launch_bounds__(kThreads) void gemv_col_kernel(GemvArgs g) {
             wv[u] = ldw<E, UNAL>(w + int64_t(k + u * KR) * g.w_ks);
             xv[u] = x[int64_t(k + u * KR) * g.x_ks];
         }
+        if constexpr (V == 8 && U == 4) {
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+            for (int e = 0; e < V; ++e) acc[e] = acc[e] + dot4<E>({wv[0][e], wv[1][e], wv[2][e], wv[3][e]}, xv);
+        } else {
 #pragma unroll
-            for (int e = 0; e < V; ++e) acc[e] = __builtin_fmaf(E::to_f32(wv[u][e]), E::to_f32(xv[u]), acc[e]);
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int e = 0; e < V; ++e) acc[e] = __builtin_fmaf(E::to_f32(wv[u][e]), E::to_f32(xv[u]), acc[e]);
+        }
     }
     for (; k < ke; k += KR) {
         const X wv = ldw<E, UNAL>(w + int64_t(k) * g.w_ks);
@@ -283,12 +346,12 @@ __global__ __launch_bounds__(kThreads) void gemv_col_kernel(GemvArgs g) {
         __syncthreads();
         for (int i = threadIdx.x; i < CL * V; i += kThreads) {
             const int c = i % CL, e = i / CL;
-            float s = red[e * CL + c];
+            typename Meet<E>::T s = red[e * CL + c];
 #pragma unroll
             for (int r = 1; r < KR; ++r) s = s + red[(r * V + e) * CL + c];
             const int own = (tile * CL + c) * V;
             const int n = min(own, g.N - V) + e;
-            if (own < g.N && n >= own) out[int64_t(n) * o_ns] = s;
+            if (own < g.N && n >= own) out[int64_t(n) * o_ns] = float(s);
         }
     }
 }

@@ -111,3 +111,31 @@ def test_short_workspace_is_refused():
     assert lib.pe_gemm(ctypes.byref(cd), *args, ctypes.c_int64(need - 1), st) == -4
     assert lib.pe_gemm(ctypes.byref(cd), *args, ctypes.c_int64(need), st) == 0
     assert float(out) == K
+
+
+@pytest.mark.parametrize("eq,s0,s1", [("ij,j->i", (500, 32), (32,)), ("ij,j->i", (3, 29), (29,)),
+                                      ("bi,bi->b", (300, 31), (300, 31)), ("bhd,bthd->bht", (2, 3, 9), (2, 70, 3, 9))])
+def test_float16_short_rows_round_once(eq, s0, s1):
+    """K <= 32: products and sums in 64 bits, one rounding to float32."""
+    a, b = _rand(s0, torch.float16, 9), _rand(s1, torch.float16, 10)
+    got, want = einsum(eq, a, b), torch.einsum(eq, a.double(), b.double())
+    mag = torch.einsum(eq, a.double().abs(), b.double().abs())
+    assert bool(((got.double() - want).abs() <= EPS * want.abs() + 2.0 ** -45 * mag).all())
+
+
+@pytest.mark.parametrize("eq,s0,s1", [("bhd,bthd->bht", (4, 8, 64), (4, 500, 8, 64)),
+                                      ("bhd,bthd->bht", (4, 8, 200), (4, 500, 8, 200)),
+                                      ("i,ij->j", (512,), (512, 4096)), ("ij,j->i", (4096, 4096), (4096,))])
+def test_float16_error_is_no_larger_than_the_tiles(eq, s0, s1):
+    """Against 64 bits, next to the same sums as a product with two equal
+    vectors (M or N of 2: matrix cores)."""
+    a, b = _rand(s0, torch.float16, 11), _rand(s1, torch.float16, 12)
+    want = torch.einsum(eq, a.double(), b.double())
+    l, r = eq.split("->")[0].split(",")
+    o = eq.split("->")[1]
+    if len(l) <= len(r):
+        two = einsum(l + "z," + r + "->" + o + "z", torch.stack([a, a], -1), b)
+    else:
+        two = einsum(l + "," + r + "z->" + o + "z", a, torch.stack([b, b], -1))
+    e = [float((x.double() - want).norm() / want.norm()) for x in (einsum(eq, a, b), two[..., 0])]
+    assert e[0] <= e[1], e
