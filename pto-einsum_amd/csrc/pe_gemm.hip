@@ -553,6 +553,23 @@ bool res_auto(const pe_gemm_desc& d, const GemmChoice& ch, bool dl, int al, int 
            gemm_res_resident(d.dtype, al, bl) >= 1;
 }
 
+// d with the roles of its operands exchanged (C' = B' A') where that makes the
+// output contiguous along N, the axis that a wave's stores run along: plans
+// that make a free axis a batch axis can ask for either (f32 abc,cd->adb 64 x
+// 512 x 256 x 512, every lane of a store on a line of its own, 375 us, 90 with
+// ordinary stores; exchanged 58).  The sums and their order stay the same.
+bool exchanged(const pe_gemm_desc& d, pe_gemm_desc& x) {
+    if (d.tile != 0 || d.split_k != 0 || d.c_ms != 1 || d.c_ns == 1 || d.M == 1 || d.N == 1) return false;
+    x = d;
+    std::swap(x.M, x.N);
+    std::swap(x.a_ms, x.b_ns);
+    std::swap(x.a_ks, x.b_ks);
+    std::swap(x.c_ms, x.c_ns);
+    std::swap(x.a_numel, x.b_numel);
+    for (int i = 0; i < d.nbatch; ++i) std::swap(x.a_bstride[i], x.b_bstride[i]);
+    return true;
+}
+
 // Store flavour of d's output (nt_mode), but ordinary stores where its rows do
 // not start on 64-byte halves of a line: neighbouring tiles then share halves,
 // which non-temporal stores write out in parts and ordinary ones join in L2.
@@ -725,6 +742,12 @@ extern "C" int pe_gemm_choice(const pe_gemm_desc* d, int64_t* info) {
     if (!d || !info) return pe::fail(PE_ERR_INVALID, "gemm_choice: null argument");
     const int st = pe::validate_gemm(*d);
     if (st != PE_OK) return st;
+    pe_gemm_desc x;
+    if (pe::exchanged(*d, x)) {
+        const int rc = pe_gemm_choice(&x, info);
+        std::swap(info[0], info[1]);
+        return rc;
+    }
     const int64_t nb = pe::batch_total(*d);
     if (nb > 0 && d->K > 0) {
         const pe::GemvPlan v = pe::gemv_plan(*d, nb);
@@ -773,6 +796,8 @@ extern "C" int pe_gemm_choice(const pe_gemm_desc* d, int64_t* info) {
 extern "C" int64_t pe_gemm_workspace_bytes(const pe_gemm_desc* d) {
     if (!d || pe::validate_gemm(*d) != PE_OK) return 0;
     if (d->K == 0 || d->M == 0 || d->N == 0 || pe::batch_total(*d) == 0) return 0;
+    pe_gemm_desc x;
+    if (pe::exchanged(*d, x)) d = &x;
     const pe::GemvPlan v = pe::gemv_plan(*d, pe::batch_total(*d));
     if (v.kind) return v.ws_bytes;
     // (float32: the register-staged kernel's own split; its choice for
@@ -792,6 +817,11 @@ extern "C" int pe_gemm(const pe_gemm_desc* d, const void* a, const void* b, floa
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t nb = batch_total(*d);
     if (nb == 0 || d->M == 0 || d->N == 0) return PE_OK;
+    pe_gemm_desc x;
+    if (exchanged(*d, x)) {
+        d = &x;
+        std::swap(a, b);
+    }
 
     ReduceArgs r{};
     r.c = c;
