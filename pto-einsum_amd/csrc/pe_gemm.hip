@@ -578,7 +578,8 @@ bool exchanged(const pe_gemm_desc& d, pe_gemm_desc& x) {
 // 5312 25.9 against 27.5), f16 4 x 16 heads 1000 x 64 x 1001 214.8 -> 98.9, f32
 // 224.8 -> 124.0.
 int store_flavour(const pe_gemm_desc& d, const float* c, int64_t nb) {
-    const int mode = nt_mode(nb * d.M * d.N * 4);
+    const int all = nt_mode(nb * d.M * d.N * 4);
+    const int mode = all == 2 && d.K <= 512 && d.c_ms == d.N ? 1 : all;
     bool lines = aligned(c, 64) && d.c_ns == 1 && d.c_ms % 16 == 0;
     for (int i = 0; i < d.nbatch; ++i) lines = lines && d.c_bstride[i] % 16 == 0;
     return lines ? mode : 0;

@@ -29,3 +29,12 @@ def test_rows_on_and_off_lines(eq, shapes, dtype):
     assert got.numel() * 4 >= 32 << 20
     want, mag = (torch.einsum(eq, x, y) for x, y in ((a.double(), b.double()), (a.double().abs(), b.double().abs())))
     assert bool(((got.double() - want).abs() <= K * EPS * mag).all())
+
+
+@pytest.mark.parametrize("eq,shapes", [
+    ("ij,jk->ik", ((8200, 32), (32, 8192))), ("ij,kj->ik", ((8200, 520), (8192, 520))),       # short and long K
+    ("bhsd,bhtd->bhst", ((1, 17, 2048, 64), (1, 17, 2048, 64))),
+])
+def test_outputs_beyond_the_last_level_cache(eq, shapes):
+    """At least 256 MB: either scope of non-temporal store."""
+    test_rows_on_and_off_lines(eq, shapes, torch.float16)
