@@ -35,7 +35,7 @@
 // Measured on one MI355X (cold operands): float16 2001 x 1537 x 3003 209 -> 50
 // us, 3001 x 5003 x 3011 775 -> 190; float32 4096^3 962 -> 731 us (188
 // TFLOP/s), 16 x 1000 x 777 x 1536 278-314 -> 227-233, 2001 x 1537 x 3003 258
-// -> 140.  float32 counters at 4096^3: matrix cores 63 % busy at 1.56 GHz,
+// -> 140 (before the L_MN layout's last change, below).  float32 counters at 4096^3: matrix cores 63 % busy at 1.56 GHz,
 // where the float32 kernel runs 89 % at 2.2: the part is at its power limit,
 // and the conversion's vector work costs clock.  Tried: the compiler's own
 // schedule 770 us, no low accumulators (64 registers fewer, no gain, errors as
@@ -185,9 +185,16 @@ struct RsOperand {
     // Element offset of (r, k) in a plane.  L_K: rows of 16 or 32 k, 16-byte groups
     // XORed so that the lanes of one ds_read_b128 phase (lanes 0-3, 12-15,
     // 20-23, 24-27 and 4-11, 16-19, 28-31 of each half wave, as bank-conflict
-    // counts show) fall in distinct banks; L_MN: as DlOperand's float16.
+    // counts show) fall in distinct banks.  L_MN: 16-byte group g of k row k at
+    // g ^ (KSWZ (k % 4)); with 16 groups a row (128 rows) 4 keeps the 32 lanes
+    // of a ds_read_b64_tr_b16 phase (two groups of 16 rows, four k) in distinct
+    // banks, where DlOperand's 2, which 64-row tiles keep, puts both groups of
+    // rows on the same ones: float32 16 x 1000 x 777 x 1536, 1.5 -> 0 conflict
+    // cycles per LDS instruction, 222.3 -> 219.0 us, float16 2001 x 1537 x 3003
+    // 43.6 -> 43.3.
+    static constexpr int KSWZ = ROWS == 128 ? 4 : 2;
     __device__ __forceinline__ static int at(int r, int k) {
-        if constexpr (LAYOUT == L_MN) return k * ROWS + (((r >> 3) ^ (2 * (k & 3))) << 3) + (r & 7);
+        if constexpr (LAYOUT == L_MN) return k * ROWS + (((r >> 3) ^ (KSWZ * (k & 3))) << 3) + (r & 7);
         else if constexpr (BK == 16) return r * 16 + (((k >> 3) ^ ((r >> 3) & 1)) << 3) + (k & 7);
         else return (k >> 5) * ROWS * 32 + r * 32 + ((((k & 31) >> 3) ^ ((r >> 2) & 3)) << 3) + (k & 7);
     }
@@ -196,7 +203,14 @@ struct RsOperand {
     // (rows 32 i .. 32 i + 31 of the wave, which starts at wrow0), MFMA step
     // st: 8 k of one row per lane.
     __device__ __forceinline__ static typename L::LaneOff lane_off(int lane, int wrow0) {
-        if constexpr (LAYOUT == L_MN) {
+        if constexpr (LAYOUT == L_MN && KSWZ == 4) {
+            // As DlOperand's, o[i] for fragment block i of a 64-row wave.
+            const int G = lane >> 4, j = (lane & 15) >> 2, q = lane & 3;
+            typename L::LaneOff x;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) x.o[i] = at(wrow0 + 32 * i + 16 * (G & 1) + 4 * q, 8 * (G >> 1) + j);
+            return x;
+        } else if constexpr (LAYOUT == L_MN) {
             return L::lane_off(lane, wrow0);
         } else {
             typename L::LaneOff x;
@@ -209,7 +223,8 @@ struct RsOperand {
                                                  int st) {
         if constexpr (LAYOUT == L_MN) {
             f16x8 v[2];
-            L::frag(plane, lo, wrow0, i, st, v);
+            if constexpr (KSWZ == 4) L::frag(plane, {{lo.o[i], lo.o[i]}}, 0, 0, st, v);
+            else L::frag(plane, lo, wrow0, i, st, v);
             return v[st % 2];
         } else {
             return *reinterpret_cast<const f16x8*>(plane + (st / 2) * ROWS * 32 + lo.o[st % 2] + i * 32 * (BK == 16 ? 16 : 32));
