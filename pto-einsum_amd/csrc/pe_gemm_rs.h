@@ -35,7 +35,7 @@
 // Measured on one MI355X (cold operands): float16 2001 x 1537 x 3003 209 -> 50
 // us, 3001 x 5003 x 3011 775 -> 190; float32 4096^3 962 -> 731 us (188
 // TFLOP/s), 16 x 1000 x 777 x 1536 278-314 -> 227-233, 2001 x 1537 x 3003 258
-// -> 140 (before the L_MN layout's last change, below).  float32 counters at 4096^3: matrix cores 63 % busy at 1.56 GHz,
+// -> 140.  float32 counters at 4096^3: matrix cores 63 % busy at 1.56 GHz,
 // where the float32 kernel runs 89 % at 2.2: the part is at its power limit,
 // and the conversion's vector work costs clock.  Tried: the compiler's own
 // schedule 770 us, no low accumulators (64 registers fewer, no gain, errors as
