@@ -10,6 +10,7 @@
 #include <string>
 
 #include "pto_einsum_hip.h"
+#include "pe_ranges.h"
 
 namespace pe {
 

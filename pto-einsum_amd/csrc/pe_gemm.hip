@@ -520,7 +520,7 @@ GemmChoice choose(const pe_gemm_desc& d, bool dl = false, int al = L_MN, int bl 
     int64_t kps = ceil_div(ceil_div(d.K, split), bk) * bk;
     split = std::max<int64_t>(1, ceil_div(d.K, kps));
     c.nsplit = int(split);
-    c.k_per_split = int(kps);
+    c.k_per_split = int(std::min<int64_t>(kps, INT32_MAX));  // (unsplit K in the last slab below 2^31)
     c.ws_bytes = split > 1 ? split * c.nbatch_total * d.M * d.N * int64_t(sizeof(float)) : 0;
     return c;
 }

@@ -167,7 +167,7 @@ __global__ __launch_bounds__(kThreads) void gemv_row_kernel(GemvArgs g) {
     if (row0 >= nrows) return;
 
     const int kb = int(blockIdx.y) * g.k_per_split;
-    const int klen = min(g.K, kb + g.k_per_split) - kb;
+    const int klen = k_range(g.K, kb, g.k_per_split);
     const T* wp[R];
     const T* xp[XROW ? R : 1];
     int64_t oo = 0;
@@ -229,10 +229,12 @@ __global__ __launch_bounds__(kThreads) void gemv_row_kernel(GemvArgs g) {
             for (int i = 0; i < R; ++i) acc[i][0] = dot16<E, A>(w[i], x[XROW ? i : 0], acc[i][0]);
         }
     }
-    for (int k = nv * V + l; k < klen; k += LPR)
+    for (int t = l; t < klen - nv * V; t += LPR) {
+        const int k = nv * V + t;
 #pragma unroll
         for (int i = 0; i < R; ++i)
             acc[i][0] = mad<E, A>(wp[i][k], xp[XROW ? i : 0][k], acc[i][0]);
+    }
 
     using M = typename Meet<E>::T;
     M s[R];
@@ -298,15 +300,16 @@ __global__ __launch_bounds__(kThreads) void gemv_col_kernel(GemvArgs g) {
     // vector owns too are summed twice and stored once.
     const int n_own = (tile * CL + col) * V;
     const int n0 = min(n_own, g.N - V);
-    const int kb = int(blockIdx.y) * g.k_per_split;
-    const int ke = min(g.K, kb + g.k_per_split);
+    // (unsigned: k may step past an end just below 2^31)
+    const uint32_t kb = blockIdx.y * uint32_t(g.k_per_split);
+    const uint32_t ke = kb + uint32_t(k_range(g.K, int32_t(kb), g.k_per_split));
     const T* w = static_cast<const T*>(g.w) + wo + n0;
     const T* x = static_cast<const T*>(g.x) + xo;
 
     float acc[V];
 #pragma unroll
     for (int e = 0; e < V; ++e) acc[e] = 0.0f;
-    int k = kb + kr;
+    uint32_t k = kb + kr;
     for (; k + (U - 1) * KR < ke; k += U * KR) {
         X wv[U];
         T xv[U];

@@ -1,0 +1,21 @@
+// Extents and launch limits that must hold up to the largest accepted sizes.
+// Plain constexpr functions (usable in kernels, on the host and in a host
+// compiler's test of them).
+#pragma once
+
+#include <cstdint>
+
+namespace pe {
+
+// k of the range that starts at kb, of at most `per`.  K may be any int32:
+// the last range's kb + per can pass 2^31 (a dot product of 2^31 - 100000
+// float16 values: 1024 ranges of 2^21), so that sum is never formed.
+constexpr int32_t k_range(int32_t K, int32_t kb, int32_t per) { return K - kb < per ? K - kb : per; }
+
+// Slabs of bk k that cover len (>= 0): as a signed sum, len + bk - 1 can pass
+// 2^31 too.
+constexpr int32_t k_slabs(int32_t len, int32_t bk) {
+    return int32_t((uint32_t(len) + uint32_t(bk) - 1u) / uint32_t(bk));
+}
+
+}  // namespace pe

@@ -1,0 +1,58 @@
+"""K ranges and slab counts of the kernels (pe_ranges.h, the header that they
+include, built here for the CPU) at extents up to the largest that descriptors
+accept, with the splits that the library chooses for them."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+from pto_einsum import abi, launch
+
+CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "pto-einsum_amd", "csrc")
+TOP = 2 ** 31 - 1
+
+
+@pytest.fixture(scope="module")
+def ranges(tmp_path_factory):
+    d = tmp_path_factory.mktemp("ranges")
+    src, lib = d / "ranges.cpp", d / "libranges.so"
+    src.write_text('#include "pe_ranges.h"\nextern "C" {\n'
+                   "int k_range(int K, int kb, int per) { return pe::k_range(K, kb, per); }\n"
+                   "int k_slabs(int len, int bk) { return pe::k_slabs(len, bk); }\n}\n")
+    # -fwrapv: 32-bit sums wrap, as they do on the GPU.
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fwrapv", "-shared", "-fPIC", f"-I{CSRC}", str(src), "-o", str(lib)],
+                   check=True)
+    return ctypes.CDLL(str(lib))
+
+
+def _choice(M, N, K, dtype, bl="k", split_k=0, tile=0):
+    d = launch.GemmDesc(dtype=dtype, batch_shape=[], a_bstride=[], b_bstride=[], c_bstride=[], M=M, N=N, K=K,
+                        a_ms=K, a_ks=1, b_ks=1 if bl == "k" else N, b_ns=K if bl == "k" else 1, c_ms=N, c_ns=1,
+                        a_numel=M * K, b_numel=K * N, c_numel=M * N, split_k=split_k, tile=tile)
+    info = (ctypes.c_int64 * 4)()
+    assert abi.bind().pe_gemm_choice(ctypes.byref(abi.gemm_desc(d)), info) == 0
+    return list(info)
+
+
+@pytest.mark.parametrize("dtype", [launch.DT_F32, launch.DT_F16])
+@pytest.mark.parametrize("K", [TOP, TOP - 7, 2 ** 31 - 64, 2 ** 31 - 100000, 2 ** 31 - 262145, 2 ** 31 - 524289,
+                               2 ** 30 + 1, 1000003, 4096, 77])
+@pytest.mark.parametrize("M,N,bl,split_k,tile", [
+    (1, 1, "k", 0, 0),       # a dot product: up to 1024 ranges
+    (1, 8, "n", 0, 0),       # vector times matrix
+    (2, 3, "k", 0, 0),       # matrix cores
+    (2, 3, "k", 1, 0), (2, 3, "k", 7, 64), (200, 200, "n", 1, 128),
+])
+def test_k_ranges_tile_the_contraction(ranges, M, N, bl, split_k, tile, K, dtype):
+    _, _, split, per = _choice(M, N, K, dtype, bl, split_k, tile)
+    assert 1 <= split and 0 < per <= TOP
+    at = 0
+    for s in range(split):
+        assert s * per == at <= TOP                  # the kernels' 32-bit start
+        n = ranges.k_range(K, s * per, per)
+        assert 0 < n <= per
+        for bk in (16, 32, 64):
+            assert ranges.k_slabs(n, bk) == -(-n // bk)
+        at += n
+    assert at == K
