@@ -123,7 +123,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(ReduceArgs r) {
     using V = typename Pack<VEC, float>::type;
     const uint32_t nv = r.per_split / VEC;
     const uint32_t stride = gridDim.x * 256;
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < nv; i += stride) {
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < nv; i = next_index(i, stride, nv)) {
         float acc[VEC];
 #pragma unroll
         for (int e = 0; e < VEC; ++e) acc[e] = 0.0f;

@@ -18,4 +18,8 @@ constexpr int32_t k_slabs(int32_t len, int32_t bk) {
     return int32_t((uint32_t(len) + uint32_t(bk) - 1u) / uint32_t(bk));
 }
 
+// The index after i of a walk over n (i < n) in steps of `stride`, n at its
+// end: i + stride can pass 2^32.
+constexpr uint32_t next_index(uint32_t i, uint32_t stride, uint32_t n) { return n - i > stride ? i + stride : n; }
+
 }  // namespace pe

@@ -19,11 +19,14 @@ def ranges(tmp_path_factory):
     src, lib = d / "ranges.cpp", d / "libranges.so"
     src.write_text('#include "pe_ranges.h"\nextern "C" {\n'
                    "int k_range(int K, int kb, int per) { return pe::k_range(K, kb, per); }\n"
-                   "int k_slabs(int len, int bk) { return pe::k_slabs(len, bk); }\n}\n")
+                   "int k_slabs(int len, int bk) { return pe::k_slabs(len, bk); }\n"
+                   "unsigned next_index(unsigned i, unsigned s, unsigned n) { return pe::next_index(i, s, n); }\n}\n")
     # -fwrapv: 32-bit sums wrap, as they do on the GPU.
     subprocess.run(["g++", "-std=c++17", "-O1", "-fwrapv", "-shared", "-fPIC", f"-I{CSRC}", str(src), "-o", str(lib)],
                    check=True)
-    return ctypes.CDLL(str(lib))
+    lib = ctypes.CDLL(str(lib))
+    lib.next_index.restype = ctypes.c_uint32
+    return lib
 
 
 def _choice(M, N, K, dtype, bl="k", split_k=0, tile=0):
@@ -56,3 +59,14 @@ def test_k_ranges_tile_the_contraction(ranges, M, N, bl, split_k, tile, K, dtype
             assert ranges.k_slabs(n, bk) == -(-n // bk)
         at += n
     assert at == K
+
+
+@pytest.mark.parametrize("n", [2 ** 32 - 1, 2 ** 32 - 2 ** 19, 2 ** 32 - 2 ** 19 - 1, 2 ** 19, 2 ** 19 + 1, 5])
+def test_strided_walks_end(ranges, n):
+    stride = 2048 * 256
+    for first in (0, 3, min(n, stride) - 1):
+        last = first + (n - 1 - first) // stride * stride if first < n else first
+        if first < n:
+            assert ranges.next_index(ctypes.c_uint32(last), ctypes.c_uint32(stride), ctypes.c_uint32(n)) == n
+        if last > first:
+            assert ranges.next_index(ctypes.c_uint32(first), ctypes.c_uint32(stride), ctypes.c_uint32(n)) == first + stride
