@@ -844,6 +844,26 @@ extern "C" int pe_gemm(const pe_gemm_desc* d, const void* a, const void* b, floa
         return PE_OK;
     }
 
+    // An axis that ends within a tile of 2^31 runs in two parts (of the same
+    // sums; neither needs more workspace than the whole).
+    const int64_t pm = axis_part(d->M), pn = axis_part(d->N), eb = d->dtype == PE_F32 ? 4 : 2;
+    if ((pm < d->M || pn < d->N) && (nb * d->M * d->N < (int64_t(1) << 32) || choose(*d).nsplit == 1)) {
+        pe_gemm_desc part = *d;
+        int64_t& ext = pm < d->M ? part.M : part.N;
+        const int64_t n0 = pm < d->M ? pm : pn;
+        const int64_t ao = pm < d->M ? n0 * d->a_ms : 0, bo = pm < d->M ? 0 : n0 * d->b_ns;
+        const int64_t co = n0 * (pm < d->M ? d->c_ms : d->c_ns), rest = ext - n0;
+        ext = n0;
+        const int rc = pe_gemm(&part, a, b, c, ws, ws_bytes, stream);
+        if (rc != PE_OK) return rc;
+        ext = rest;
+        part.a_numel -= ao;
+        part.b_numel -= bo;
+        part.c_numel -= co;
+        return pe_gemm(&part, static_cast<const char*>(a) + ao * eb, static_cast<const char*>(b) + bo * eb, c + co, ws,
+                       ws_bytes, stream);
+    }
+
     const GemvPlan v = gemv_plan(*d, nb);
     if (v.kind) {  // a matrix-vector product
         if (v.ws_bytes > 0 && (!ws || ws_bytes < v.ws_bytes))

@@ -18,6 +18,11 @@ constexpr int32_t k_slabs(int32_t len, int32_t bk) {
     return int32_t((uint32_t(len) + uint32_t(bk) - 1u) / uint32_t(bk));
 }
 
+// Rows (or columns) of a GEMM that run in one launch, the rest in another:
+// the kernels form the end of a tile (at most 256 rows) in 32 bits, and an
+// axis that ends within a tile of 2^31 would end at 2^31.
+constexpr int64_t axis_part(int64_t n) { return n > (int64_t(1) << 31) - 256 ? int64_t(1) << 30 : n; }
+
 // The index after i of a walk over n (i < n) in steps of `stride`, n at its
 // end: i + stride can pass 2^32.
 constexpr uint32_t next_index(uint32_t i, uint32_t stride, uint32_t n) { return n - i > stride ? i + stride : n; }

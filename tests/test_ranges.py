@@ -20,12 +20,13 @@ def ranges(tmp_path_factory):
     src.write_text('#include "pe_ranges.h"\nextern "C" {\n'
                    "int k_range(int K, int kb, int per) { return pe::k_range(K, kb, per); }\n"
                    "int k_slabs(int len, int bk) { return pe::k_slabs(len, bk); }\n"
+                   "int64_t axis_part(int64_t n) { return pe::axis_part(n); }\n"
                    "unsigned next_index(unsigned i, unsigned s, unsigned n) { return pe::next_index(i, s, n); }\n}\n")
     # -fwrapv: 32-bit sums wrap, as they do on the GPU.
     subprocess.run(["g++", "-std=c++17", "-O1", "-fwrapv", "-shared", "-fPIC", f"-I{CSRC}", str(src), "-o", str(lib)],
                    check=True)
     lib = ctypes.CDLL(str(lib))
-    lib.next_index.restype = ctypes.c_uint32
+    lib.next_index.restype, lib.axis_part.restype = ctypes.c_uint32, ctypes.c_int64
     return lib
 
 
@@ -59,6 +60,15 @@ def test_k_ranges_tile_the_contraction(ranges, M, N, bl, split_k, tile, K, dtype
             assert ranges.k_slabs(n, bk) == -(-n // bk)
         at += n
     assert at == K
+
+
+@pytest.mark.parametrize("n", [TOP, TOP - 7, 2 ** 31 - 128, 2 ** 31 - 255, 2 ** 31 - 256, 2 ** 31 - 257, 2 ** 30, 1])
+def test_tiles_of_a_launch_end_below_the_32_bit_range(ranges, n):
+    first = ranges.axis_part(ctypes.c_int64(n))
+    assert 0 < first <= n
+    for part in {first, n - first}:
+        for tile in (32, 64, 128, 192, 256):
+            assert -(-part // tile) * tile <= TOP
 
 
 @pytest.mark.parametrize("n", [2 ** 32 - 1, 2 ** 32 - 2 ** 19, 2 ** 32 - 2 ** 19 - 1, 2 ** 19, 2 ** 19 + 1, 5])
