@@ -62,7 +62,7 @@ class EinsumBuilder:
         self.code_hash: Optional[str] = None
         self.target_dir: Optional[str] = None
         self.launch_plan: Optional[launch.LaunchPlan] = None
-        self._workspaces: Dict[int, tuple] = {}   # device -> (workspace tensor, its allocation stream)
+        self._workspaces: Dict[tuple, torch.Tensor] = {}   # (device, stream, thread) -> workspace
         self._swap_operands = False
         self._exec_shapes = tuple(tuple(s) for s in input_shapes)
         self._exec_equation: Optional[str] = None
@@ -155,10 +155,10 @@ class EinsumBuilder:
 
     # --- lifecycle (builder.py:738-759) ----------------------------------
     def _free_workspaces(self):
-        # The runner's workspaces are torch allocations: dropping them returns
-        # the memory to torch's stream-ordered caching allocator, which hands
-        # it out again only behind the work already queued on the streams
-        # that used it (recorded in run()).  No device synchronisation.
+        # The runner's workspaces are torch allocations, each used on the
+        # stream it was allocated on only: dropping them returns the memory to
+        # torch's stream-ordered caching allocator, which hands it out again
+        # behind the work already queued there.  No device synchronisation.
         self._workspaces = {}
 
     def cleanup(self):
@@ -166,6 +166,19 @@ class EinsumBuilder:
         self.lib = None
         if self.target_dir and os.path.exists(self.target_dir):
             shutil.rmtree(self.target_dir)
+
+    def _workspace(self, key, dev):
+        """A workspace for launches of one host thread on one stream (``key``
+        = device, stream, thread): calls on other streams, or another thread's
+        between the kernels of one call, would write the same partials.  The
+        first _KEPT_WORKSPACES of a runner are kept for the next call; further
+        ones, and those of a call under graph capture, which belong to the
+        graph's own memory pool, last for the call (torch's allocator reuses
+        them in stream order)."""
+        ws = torch.empty(self._ws_bytes, dtype=torch.uint8, device=dev)
+        if len(self._workspaces) < _KEPT_WORKSPACES and not _capturing():
+            self._workspaces[key] = ws
+        return ws
 
     # --- runner (builder.py:817-884) -------------------------------------
     def _ptr(self, t: torch.Tensor, ctype):
@@ -180,7 +193,11 @@ class EinsumBuilder:
         if gpu:
             from . import abi
 
-            self._ws_bytes = int(abi.bind().pe_einsum_workspace_bytes(ctypes.byref(abi.einsum_plan(self.launch_plan))))
+            lib, p, plan = abi.bind(), self.launch_plan, abi.einsum_plan(self.launch_plan)
+            self._ws_bytes = int(lib.pe_einsum_workspace_bytes(ctypes.byref(plan)))
+            uses_ws = p.route == launch.ROUTE_GEMM and (p.gather0 or p.gather1 or p.scatter_out or
+                                                        lib.pe_gemm_workspace_bytes(ctypes.byref(plan.gemm)) > 0)
+            capturing, thread = torch.cuda.is_current_stream_capturing, threading.get_ident
 
         # The call's constants, and the C entry with plain pointers (the
         # library object's own attribute keeps the reference's argtypes).
@@ -197,19 +214,12 @@ class EinsumBuilder:
             dev = inp0.device
             out = torch.empty(out_shape, dtype=torch.float32, device=dev)
             stream = runtime.raw_stream(idx)
-            # Workspace (split-K partials, staged operands): a torch
-            # allocation per device, so creating it is stream-ordered and
-            # allowed under graph capture, and dropping it needs no
-            # synchronisation.  A use on another stream than the one it was
-            # allocated on is recorded, so the allocator does not reuse the
-            # memory before that stream's work is done.
-            entry = self._workspaces.get(idx)
-            if entry is None:
-                entry = (torch.empty(self._ws_bytes, dtype=torch.uint8, device=dev), stream)
-                self._workspaces[idx] = entry
-            elif entry[1] != stream:
-                entry[0].record_stream(torch.cuda.current_stream(dev))
-            rc = exec_fn(inp0.data_ptr(), inp1.data_ptr(), out.data_ptr(), entry[0].data_ptr(), stream)
+            # A workspace that no kernel touches may be anyone's.
+            key = (idx, stream, thread()) if uses_ws else (idx, 0, 0)
+            ws = self._workspaces.get(key)
+            if ws is None or (uses_ws and capturing()):
+                ws = self._workspace(key, dev)
+            rc = exec_fn(inp0.data_ptr(), inp1.data_ptr(), out.data_ptr(), ws.data_ptr(), stream)
             if rc:
                 runtime.check(rc, "run_einsum_exec")
             return out
@@ -254,11 +264,12 @@ class EinsumBuilder:
 
 
 _RUNNER_CACHE_SIZE = 64
+# Workspaces that one runner keeps, each for a stream and thread of its own.
+_KEPT_WORKSPACES = 8
 _runners: "collections.OrderedDict" = collections.OrderedDict()
 _runners_lock = threading.Lock()
-# Runners handed out while a StageGraph captures: the graph keeps them (and so
-# their workspaces, which its replays read and write) alive after the cache
-# evicts them.  None outside a capture.
+# Runners handed out while a StageGraph captures: the graph keeps them alive
+# after the cache evicts them.  None outside a capture.
 _capture_pins: Optional[list] = None
 
 
@@ -350,9 +361,9 @@ def einsum(equation: str, *operands, device: str = "cuda", reduce_solo_axes: boo
 def _use_runner(key, entry) -> None:
     """Cache upkeep of a call that uses ``entry`` (the lock is held)."""
     _runners.move_to_end(key)
-    # No eviction while a graph is being captured: a runner used earlier in
-    # the capture must keep its workspace, which the graph reads at every
-    # replay.  The cache shrinks back at the first call after it.
+    # No eviction while a graph is being captured (what a capture uses stays
+    # until its graph holds it).  The cache shrinks back at the first call
+    # after it.
     if len(_runners) > _RUNNER_CACHE_SIZE and not _capturing():
         while len(_runners) > _RUNNER_CACHE_SIZE:
             _runners.popitem(last=False)

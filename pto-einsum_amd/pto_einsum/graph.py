@@ -17,10 +17,10 @@ The library's execution entry points are safe to capture: they launch kernels
 on the caller's current stream and never allocate device memory, synchronise,
 or clear memory with a memset (split-K partial sums are combined by a
 reduction kernel in a fixed order), so every replay is bit-identical to an
-eager call on the same inputs.  Runner workspaces are torch allocations
-(allowed under capture); the graph keeps every einsum runner it captured alive,
-so their workspaces outlive evictions from the runner cache, which pauses
-while a capture runs.  Building runners (host-side code generation) is best
+eager call on the same inputs.  A call under capture takes its workspace from
+the graph's own memory pool, so replays share none with eager calls or with
+other graphs; the graph keeps every einsum runner it captured alive past
+evictions from the runner cache, which pause while a capture runs.  Building runners (host-side code generation) is best
 left to the eager warm-up calls that precede the capture.
 """
 from __future__ import annotations
@@ -54,9 +54,8 @@ class StageGraph:
             torch.cuda.current_stream().wait_stream(side)
             torch.cuda.synchronize()
             self._graph = torch.cuda.CUDAGraph()
-            # Every einsum runner used in the capture is kept with the graph:
-            # its workspace is part of what the replays read and write, so it
-            # must outlive the runner cache's eviction of that runner.
+            # Every einsum runner used in the capture is kept with the graph,
+            # past the runner cache's eviction of it.
             prev = builder._capture_pins
             builder._capture_pins = []
             try:
