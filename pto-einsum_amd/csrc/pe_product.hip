@@ -583,8 +583,8 @@ hipError_t launch_rows(const ProductArgs& args, uint32_t n, bool add_zero, hipSt
 }
 
 // Launches product_tile_kernel if the second operand (or, swapped, the first)
-// runs along an outer axis of at least 8, as the output's inner axis is;
-// false: not such a product.
+// runs along an outer axis of at least 8, as the output's inner axis is, and
+// the tiles are full enough (product_tile_blocks); false: not such a product.
 template <typename E>
 bool launch_tiles(const ProductArgs& args, const std::vector<int64_t>& shape, bool add_zero, hipStream_t s,
                   hipError_t& e) {
@@ -627,12 +627,12 @@ bool launch_tiles(const ProductArgs& args, const std::vector<int64_t>& shape, bo
         batches *= shape[k];
         ++g.nbatch;
     }
-    const int64_t tiles = int64_t(g.tiles_p) * ceil_div(shape[q], kPT);
-    if (tiles * batches >= (int64_t(1) << 31)) return false;
-    g.tiles = uint32_t(tiles);
+    const int64_t blocks = product_tile_blocks(P, shape[q], batches);
+    if (blocks == 0 || blocks >= (int64_t(1) << 31)) return false;
+    g.tiles = uint32_t(blocks / batches);
     g.nt = args.nt;
     const bool aq = g.a_p > 1 && g.a_q == 1;
-    const dim3 grid(uint32_t(tiles * batches));
+    const dim3 grid{uint32_t(blocks)};
     if (aq && add_zero) hipLaunchKernelGGL((product_tile_kernel<E, true, true>), grid, dim3(kThreads), 0, s, g);
     else if (aq) hipLaunchKernelGGL((product_tile_kernel<E, true, false>), grid, dim3(kThreads), 0, s, g);
     else if (add_zero) hipLaunchKernelGGL((product_tile_kernel<E, false, true>), grid, dim3(kThreads), 0, s, g);

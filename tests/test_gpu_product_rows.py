@@ -68,3 +68,10 @@ def test_rows_bit_exact(shape, sa, sb, off, add_zero, dtype):
     got = out.cpu()
     assert bool(torch.isnan(got[n:]).all())
     assert torch.equal(got[:n].view(torch.int32), want.contiguous().view(-1).view(torch.int32))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("nb,q,p", [(1000, 8, 8), (300, 12, 12), (300, 15, 17), (300, 16, 16), (40, 64, 8), (40, 8, 64)])
+def test_many_small_transposed_matrices(nb, q, p, dtype):
+    """bqp,bpq->bqp on both sides of the tile kernel's rule on full tiles."""
+    test_rows_bit_exact((nb, q, p), (q * p, p, 1), (q * p, 1, q), 0, 0, dtype)

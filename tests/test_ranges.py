@@ -20,6 +20,8 @@ def ranges(tmp_path_factory):
     src.write_text('#include "pe_ranges.h"\nextern "C" {\n'
                    "int k_range(int K, int kb, int per) { return pe::k_range(K, kb, per); }\n"
                    "int k_slabs(int len, int bk) { return pe::k_slabs(len, bk); }\n"
+                   "int64_t product_tile_blocks(int64_t P, int64_t Q, int64_t b)"
+                   " { return pe::product_tile_blocks(P, Q, b); }\n"
                    "int64_t axis_part(int64_t n) { return pe::axis_part(n); }\n"
                    "unsigned next_index(unsigned i, unsigned s, unsigned n) { return pe::next_index(i, s, n); }\n}\n")
     # -fwrapv: 32-bit sums wrap, as they do on the GPU.
@@ -27,6 +29,8 @@ def ranges(tmp_path_factory):
                    check=True)
     lib = ctypes.CDLL(str(lib))
     lib.next_index.restype, lib.axis_part.restype = ctypes.c_uint32, ctypes.c_int64
+    lib.product_tile_blocks.restype = ctypes.c_int64
+    lib.product_tile_blocks.argtypes = [ctypes.c_int64] * 3
     return lib
 
 
@@ -80,3 +84,12 @@ def test_strided_walks_end(ranges, n):
             assert ranges.next_index(ctypes.c_uint32(last), ctypes.c_uint32(stride), ctypes.c_uint32(n)) == n
         if last > first:
             assert ranges.next_index(ctypes.c_uint32(first), ctypes.c_uint32(stride), ctypes.c_uint32(n)) == first + stride
+
+
+@pytest.mark.parametrize("P,Q,batches,want", [
+    (4096, 4096, 1, 4096), (1001, 1003, 3, 768), (16, 16, 1000, 1000), (8, 64, 7, 7), (8, 1024, 7, 112),
+    (65, 65, 2, 8), (8, 65, 1, 2),
+    (8, 8, 1 << 20, 0), (12, 12, 1000, 0), (15, 17, 3, 0), (9, 513, 1, 9), (8, 31, 5, 0),     # mostly empty tiles
+])
+def test_product_tiles_are_filled(ranges, P, Q, batches, want):
+    assert ranges.product_tile_blocks(P, Q, batches) == want
