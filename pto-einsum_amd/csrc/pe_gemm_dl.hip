@@ -84,7 +84,7 @@ hipError_t launch_gemm_dl(int dtype, int bm, int bn, int minb, int al, int bl, b
     const int resident = gemm_dl_resident(dtype, bm, bn, minb, al, bl);
     if (resident < 1) return hipErrorInvalidConfiguration;
     GemmArgs a = g;
-    const uint32_t cap = persist ? uint32_t(cu_count()) * uint32_t(resident) : 0x7fffffffu;
+    const uint32_t cap = persist ? uint32_t(cu_count()) * uint32_t(resident) : uint32_t(kMaxBlocks);
     if (a.grid > cap) a.grid = cap;
     void* args[] = {&a};
     return hipLaunchKernel(dl_kernel(dtype, bm, bn, minb, al, bl), dim3(a.grid), dim3(kGemmThreads), args, 0, s);

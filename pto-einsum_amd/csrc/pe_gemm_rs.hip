@@ -24,7 +24,7 @@ static const void* rs_kernel(int dtype, int tile, int al, int bl) {
 hipError_t launch_gemm_rs(int dtype, int tile, int al, int bl, const GemmArgs& g, hipStream_t s) {
     if (dtype == PE_F32 && tile != 128) return hipErrorInvalidConfiguration;
     GemmArgs a = g;
-    if (a.grid > 0x7fffffffu) a.grid = 0x7fffffffu;  // the tile walk strides over the rest
+    if (a.grid > kMaxBlocks) a.grid = uint32_t(kMaxBlocks);  // the tile walk strides over the rest
     void* args[] = {&a};
     return hipLaunchKernel(rs_kernel(dtype, tile, al, bl), dim3(a.grid), dim3(kGemmThreads), args, 0, s);
 }

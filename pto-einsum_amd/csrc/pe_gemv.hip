@@ -468,7 +468,7 @@ GemvPlan gemv_plan(const pe_gemm_desc& d, int64_t nb) {
     }
     if (p.split == 1) p.kps = int(d.K);
     p.split = int(ceil_div(d.K, p.kps));
-    if (p.blocks >= (int64_t(1) << 31)) p.kind = 0;
+    if (p.blocks > kMaxBlocks) p.kind = 0;  // (the tile kernels walk a smaller grid)
     p.ws_bytes = p.split > 1 ? int64_t(p.split) * rows * 4 : 0;
     return p;
 }

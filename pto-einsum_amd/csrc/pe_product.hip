@@ -628,7 +628,7 @@ bool launch_tiles(const ProductArgs& args, const std::vector<int64_t>& shape, bo
         ++g.nbatch;
     }
     const int64_t blocks = product_tile_blocks(P, shape[q], batches);
-    if (blocks == 0 || blocks >= (int64_t(1) << 31)) return false;
+    if (blocks == 0) return false;
     g.tiles = uint32_t(blocks / batches);
     g.nt = args.nt;
     const bool aq = g.a_p > 1 && g.a_q == 1;

@@ -27,15 +27,20 @@ constexpr int64_t axis_part(int64_t n) { return n > (int64_t(1) << 31) - 256 ? i
 // end: i + stride can pass 2^32.
 constexpr uint32_t next_index(uint32_t i, uint32_t stride, uint32_t n) { return n - i > stride ? i + stride : n; }
 
+// Blocks of 256 threads in a launch: HIP takes fewer than 2^32 threads along an
+// axis of the grid.
+constexpr int64_t kMaxBlocks = (int64_t(1) << 24) - 1;
+
 // Blocks of the product kernel's 64 x 64 tiles over `batches` matrices of P x
-// Q, or 0 where it does not serve: it moves a whole tile's elements whatever
-// part of it is there, so a matrix's tiles are at least a sixteenth full.  One
-// MI355X, one element per lane against tiles, 8.4 million outputs: 8 x 8
-// matrices f16 142 against 297 us, f32 142 / 228, 12 x 12 143 / 155 and 169 /
-// 107, 16 x 16 145 / 97 and 144 / 65, 8 x 64 142 / 51 and 145 / 34.
+// Q, or 0 where it does not serve: more than a launch holds, or tiles less
+// than a sixteenth full (it moves a whole tile's elements whatever part of it
+// is there).  One MI355X, one element per lane against tiles, 8.4 million
+// outputs: 8 x 8 matrices f16 142 against 297 us, f32 142 / 228, 12 x 12 143 /
+// 155 and 169 / 107, 16 x 16 145 / 97 and 144 / 65, 8 x 64 142 / 51 and 145 /
+// 34.
 constexpr int64_t product_tile_blocks(int64_t P, int64_t Q, int64_t batches) {
     const int64_t tiles = ((P + 63) / 64) * ((Q + 63) / 64);
-    return 16 * P * Q >= 64 * 64 * tiles ? tiles * batches : 0;
+    return 16 * P * Q >= 64 * 64 * tiles && tiles * batches <= kMaxBlocks ? tiles * batches : 0;
 }
 
 }  // namespace pe

@@ -89,7 +89,26 @@ def test_strided_walks_end(ranges, n):
 @pytest.mark.parametrize("P,Q,batches,want", [
     (4096, 4096, 1, 4096), (1001, 1003, 3, 768), (16, 16, 1000, 1000), (8, 64, 7, 7), (8, 1024, 7, 112),
     (65, 65, 2, 8), (8, 65, 1, 2),
+    (64, 64, (1 << 24) - 1, (1 << 24) - 1), (64, 64, 1 << 24, 0), (8, 65, 1 << 23, 0),    # 2^32 threads
     (8, 8, 1 << 20, 0), (12, 12, 1000, 0), (15, 17, 3, 0), (9, 513, 1, 9), (8, 31, 5, 0),     # mostly empty tiles
 ])
-def test_product_tiles_are_filled(ranges, P, Q, batches, want):
+def test_product_tiles_are_filled_and_fit_a_launch(ranges, P, Q, batches, want):
     assert ranges.product_tile_blocks(P, Q, batches) == want
+
+
+@pytest.mark.parametrize("dtype", [launch.DT_F32, launch.DT_F16])
+@pytest.mark.parametrize("nb,N,K,bl,taken", [
+    (2 ** 24 - 1, 8, 8, "n", True), (2 ** 24, 8, 8, "n", False),    # a block for each batch
+    (2 ** 24, 16, 300, "k", False), (2 ** 22 - 1, 16, 300, "k", True),    # four rows of a batch in a block
+    (2 ** 24, 2, 200, "k", True),                                         # 64 rows of any batch
+])
+def test_vector_kernels_fit_a_launch(nb, N, K, bl, taken, dtype):
+    """Grids of 2^32 threads stay on the tile kernels, which walk a smaller one."""
+    if bl == "k" and dtype == launch.DT_F32:
+        K //= 2     # the same lanes for each row
+    d = launch.GemmDesc(dtype=dtype, batch_shape=[nb], a_bstride=[K], b_bstride=[K * N], c_bstride=[N], M=1, N=N, K=K,
+                        a_ms=0, a_ks=1, b_ks=1 if bl == "k" else N, b_ns=K if bl == "k" else 1, c_ms=0, c_ns=1,
+                        a_numel=nb * K, b_numel=nb * K * N, c_numel=nb * N)
+    info = (ctypes.c_int64 * 4)()
+    assert abi.bind().pe_gemm_choice(ctypes.byref(abi.gemm_desc(d)), info) == 0
+    assert (list(info)[:2] == [1, 1]) == taken
