@@ -133,8 +133,11 @@ int pe_gemm(const pe_gemm_desc* d, const void* a, const void* b, float* c, void*
  * tests and tuning): info[0..3] = tile rows, tile columns, K splits, k per
  * split (256 x 256 for the large float16 kernel; 1, 1 for a matrix-vector
  * product, M or N = 1 and the other operand contiguous along k or its free
- * axis).  But for matrix-vector products, the split, and so the workspace
- * size, is the same for every operand layout; it never depends on addresses. */
+ * axis).  The workspace size follows from extents and strides alone, and so
+ * does the split, but where a kernel for whole aligned vectors needs none (the
+ * large float16 and the short-K kernel; small grids whose blocks split K among
+ * their waves): operands off the 16-byte grid may then take the split that the
+ * workspace is sized for. */
 int pe_gemm_choice(const pe_gemm_desc* d, int64_t* info);
 
 /* Fused linear-attention chain.  No single entry point of the reference

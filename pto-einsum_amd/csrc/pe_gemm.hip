@@ -636,7 +636,9 @@ bool rs_eligible(const pe_gemm_desc& d, int& al, int& bl) {
 
 // The register-staged kernel's tile and K split for d, if it is the one to
 // run: float16 operands that the direct-load kernels cannot take (dl false),
-// float32 ones by PE_GEMM_RS_F32_MIN_K's rule.
+// float32 ones by PE_GEMM_RS_F32_MIN_K's rule.  Where dl, and so the operands'
+// addresses, decide, the split is choose()'s: a base off the vector grid
+// changes neither the sums' lengths nor the workspace.
 bool rs_choice(const pe_gemm_desc& d, bool dl, int& al, int& bl, GemmChoice& ch) {
     if ((d.dtype == PE_F16 && dl) || !rs_eligible(d, al, bl)) return false;
     if (d.dtype == PE_F32 &&
@@ -649,12 +651,6 @@ bool rs_choice(const pe_gemm_desc& d, bool dl, int& al, int& bl, GemmChoice& ch)
         // against 19.8).
         if (16 * ch.nbatch_total * ceil_div(d.M, 128) * ceil_div(d.N, 128) * ch.nsplit <= cu_count())
             ch.bm = ch.bn = 64;
-        // Splits in whole 64-k slabs (no more of them, so the workspace of
-        // choose() holds).
-        if (ch.nsplit > 1) {
-            ch.k_per_split = int(ceil_div(ch.k_per_split, 64) * 64);
-            ch.nsplit = int(ceil_div(d.K, ch.k_per_split));
-        }
         return true;
     }
     const int64_t tiles = ch.nbatch_total * ceil_div(d.M, 128) * ceil_div(d.N, 128), cus = cu_count();
@@ -669,7 +665,7 @@ bool rs_choice(const pe_gemm_desc& d, bool dl, int& al, int& bl, GemmChoice& ch)
                (n > 1 ? 100.0 + 3.2e-5 * double(n) * double(ch.nbatch_total) * double(d.M) * double(d.N) : 0.0);
     };
     if (split && (!whole || cost(ch.nsplit, ch.k_per_split) < cost(1, d.K))) return true;
-    if (!whole) return false;
+    if (!whole || (ch.nsplit > 1 && d.K < PE_GEMM_RS_F32_MIN_K)) return false;
     ch.bm = ch.bn = 128;
     ch.nsplit = 1;
     ch.k_per_split = int(d.K);

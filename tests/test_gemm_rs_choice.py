@@ -73,3 +73,23 @@ def test_every_load_lies_in_its_operand(L, V, rows_tile, BK, rows, K):
     for kps in (K, 64):
         for addr, n in _addresses(L, V, rows_tile, BK, rows, K, kps):
             assert 0 <= addr and addr + n <= rows * K
+
+
+@pytest.mark.parametrize("dtype", [launch.DT_F16, launch.DT_F32])
+@pytest.mark.parametrize("M,N,K", [(640, 48, 1992), (768, 96, 560), (304, 200, 1000), (504, 536, 504), (4000, 128, 4104),
+                                   (264, 264, 1960), (2000, 3000, 72), (1000, 1504, 160), (2048, 2048, 512),
+                                   (1664, 1920, 1000), (136, 264, 200)])
+def test_split_does_not_depend_on_alignment(M, N, K, dtype):
+    """Operands off the vector grid (as an odd batch stride of one batch makes
+    them for the choice) are split as aligned ones are, where those are split
+    or unsplit by the same rule."""
+    infos = []
+    for odd in (0, 1):
+        d = launch.GemmDesc(dtype=dtype, batch_shape=[1], a_bstride=[M * K + odd], b_bstride=[K * N + odd],
+                            c_bstride=[M * N], M=M, N=N, K=K, a_ms=K, a_ks=1, b_ks=N, b_ns=1, c_ms=N, c_ns=1,
+                            a_numel=M * K, b_numel=K * N, c_numel=M * N)
+        lib, cd, info = abi.bind(), abi.gemm_desc(d), (ctypes.c_int64 * 4)()
+        assert lib.pe_gemm_choice(ctypes.byref(cd), info) == 0
+        infos.append(([info[2], info[3] if info[2] > 1 else K], int(lib.pe_gemm_workspace_bytes(ctypes.byref(cd)))))
+        assert infos[-1][1] >= (infos[-1][0][0] * M * N * 4 if infos[-1][0][0] > 1 else 0)
+    assert infos[0] == infos[1]
