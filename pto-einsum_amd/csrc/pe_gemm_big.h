@@ -353,7 +353,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_big_kernel(GemmArgs g) {
     const uint32_t tiles_all = g.tiles_per_batch * g.nbatch_total;
     const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(
         (const __attribute__((address_space(3))) _Float16*)(lds)));
-    const int nslabs = k_slabs(g.K, BK);                     // slabs per tile (every tile has all of K)
+    const int nslabs = (g.K + BK - 1) / BK;                  // slabs per tile (every tile has all of K)
     const int tail_slab = TAIL ? nslabs - 1 : nslabs;        // the slab with a K tail, if any
     // Byte steps of the load pointers per slab.
     const int64_t step_a = int64_t(BK) * g.a_ks, step_b = int64_t(BK) * g.b_ks;

@@ -420,8 +420,8 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_dl_kernel(GemmArgs g)
         x.m0 = tm * BM;
         x.n0 = tn * BN;
         const int kb = int(x.split) * g.k_per_split;
-        x.k_len = k_range(g.K, kb, g.k_per_split);
-        x.nslabs = k_slabs(x.k_len, BK);
+        x.k_len = min(g.K, kb + g.k_per_split) - kb;
+        x.nslabs = (x.k_len + BK - 1) / BK;
         x.rows_a = g.M - x.m0;
         x.rows_b = g.N - x.n0;
         x.A = static_cast<const T*>(g.a) + a_off + int64_t(x.m0) * g.a_ms + int64_t(kb) * g.a_ks;

@@ -71,6 +71,7 @@ bool gemm_dl_eligible(int dtype, int al, int bl, int64_t M, int64_t N, int64_t K
     if (al == L_MN && M % vec != 0) return false;
     if (bl == L_MN && N % vec != 0) return false;
     if ((al == L_K || bl == L_K) && K % vec != 0) return false;
+    if (!k_ends_fit(K)) return false;
     // 32-bit store offsets: every element of a tile (at most 256 x 256)
     // within 2^31 bytes of its corner, for the output and for the row-major
     // split-K partials (strides N and 1).

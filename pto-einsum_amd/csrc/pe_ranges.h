@@ -9,14 +9,24 @@ namespace pe {
 
 // k of the range that starts at kb, of at most `per`.  K may be any int32:
 // the last range's kb + per can pass 2^31 (a dot product of 2^31 - 100000
-// float16 values: 1024 ranges of 2^21), so that sum is never formed.
-constexpr int32_t k_range(int32_t K, int32_t kb, int32_t per) { return K - kb < per ? K - kb : per; }
+// float16 values: 1024 ranges of 2^21), so the sum is unsigned.
+constexpr int32_t k_range(int32_t K, int32_t kb, int32_t per) {
+    const uint32_t end = uint32_t(kb) + uint32_t(per);
+    return int32_t((uint32_t(K) < end ? uint32_t(K) : end) - uint32_t(kb));
+}
 
 // Slabs of bk k that cover len (>= 0): as a signed sum, len + bk - 1 can pass
 // 2^31 too.
 constexpr int32_t k_slabs(int32_t len, int32_t bk) {
     return int32_t((uint32_t(len) + uint32_t(bk) - 1u) / uint32_t(bk));
 }
+
+// Whether every range of K and every slab of it ends below 2^31, however K is
+// split (splits of whole slabs end less than 2^20 past K).  Kernels that form
+// these ends as plain sums take such K only (gemm_dl_eligible): with k_range
+// instead, the direct-load float32 64x64 tiles ran up to 9 % longer (82 x 152 x
+// 400, K = 1024, 129 -> 141 us).
+constexpr bool k_ends_fit(int64_t K) { return K <= INT32_MAX - (1 << 20); }
 
 // Rows (or columns) of a GEMM that run in one launch, the rest in another:
 // the kernels form the end of a tile (at most 256 rows) in 32 bits, and an

@@ -20,6 +20,7 @@ def ranges(tmp_path_factory):
     src.write_text('#include "pe_ranges.h"\nextern "C" {\n'
                    "int k_range(int K, int kb, int per) { return pe::k_range(K, kb, per); }\n"
                    "int k_slabs(int len, int bk) { return pe::k_slabs(len, bk); }\n"
+                   "bool k_ends_fit(int64_t K) { return pe::k_ends_fit(K); }\n"
                    "int64_t product_tile_blocks(int64_t P, int64_t Q, int64_t b)"
                    " { return pe::product_tile_blocks(P, Q, b); }\n"
                    "int64_t axis_part(int64_t n) { return pe::axis_part(n); }\n"
@@ -29,6 +30,7 @@ def ranges(tmp_path_factory):
                    check=True)
     lib = ctypes.CDLL(str(lib))
     lib.next_index.restype, lib.axis_part.restype = ctypes.c_uint32, ctypes.c_int64
+    lib.k_ends_fit.restype = ctypes.c_bool
     lib.product_tile_blocks.restype = ctypes.c_int64
     lib.product_tile_blocks.argtypes = [ctypes.c_int64] * 3
     return lib
@@ -45,6 +47,7 @@ def _choice(M, N, K, dtype, bl="k", split_k=0, tile=0):
 
 @pytest.mark.parametrize("dtype", [launch.DT_F32, launch.DT_F16])
 @pytest.mark.parametrize("K", [TOP, TOP - 7, 2 ** 31 - 64, 2 ** 31 - 100000, 2 ** 31 - 262145, 2 ** 31 - 524289,
+                               2 ** 31 - 2 ** 20 - 8,
                                2 ** 30 + 1, 1000003, 4096, 77])
 @pytest.mark.parametrize("M,N,bl,split_k,tile", [
     (1, 1, "k", 0, 0),       # a dot product: up to 1024 ranges
@@ -64,6 +67,8 @@ def test_k_ranges_tile_the_contraction(ranges, M, N, bl, split_k, tile, K, dtype
             assert ranges.k_slabs(n, bk) == -(-n // bk)
         at += n
     assert at == K
+    if ranges.k_ends_fit(ctypes.c_int64(K)):
+        assert split * per <= TOP and K + 255 <= TOP
 
 
 @pytest.mark.parametrize("n", [TOP, TOP - 7, 2 ** 31 - 128, 2 ** 31 - 255, 2 ** 31 - 256, 2 ** 31 - 257, 2 ** 30, 1])
