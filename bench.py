@@ -7,7 +7,7 @@ operands and output resident in HBM.  ``value`` is TFLOP/s over the timed
 steps (2*b*i*j*k flops per step).  ``roofline`` relates the GEMM kernel's
 average launch time (HIP events recorded around each launch on the launch
 stream) to the float32 MFMA peak (``split_peak``: the bfloat16 peak over the
-six products of terms that it forms per float32 product).  ``cpu_baseline`` times the reference CPU
+eight products of terms that it forms per float32 product).  ``cpu_baseline`` times the reference CPU
 route (cpu_einsum.h compiled by oracle/ref_build.py; the C restatement in
 oracle/ when that build is absent) on the whole of config 2, one thread, and
 every ``per_config`` row carries the same route's time on that config
@@ -412,10 +412,10 @@ def roofline(flops, nbytes, t_ms, dtype):
                     frac=round(tflops / PEAK_TFLOPS[dtype], 4))
         if dtype == "f32":
             # Longer float32 contractions multiply on bfloat16 matrix cores,
-            # six products of terms per product, and may pass the float32
+            # eight products of terms per product, and may pass the float32
             # peak: the roof of that form beside it.
-            roof["split_peak"] = round(PEAK_TFLOPS["f16"] / 6, 1)
-            roof["split_frac"] = round(tflops / (PEAK_TFLOPS["f16"] / 6), 4)
+            roof["split_peak"] = round(PEAK_TFLOPS["f16"] / 8, 1)
+            roof["split_frac"] = round(tflops / (PEAK_TFLOPS["f16"] / 8), 4)
         return roof, tflops, gbs
     return dict(bound="hbm", achieved=round(gbs, 1), peak=PEAK_HBM_GBS, unit="GB/s",
                 frac=round(gbs / PEAK_HBM_GBS, 4)), tflops, gbs

@@ -75,22 +75,22 @@
 // 128^3, one 128x128 tile per CU) it took 20.8-22.6 us against 18.9-19.6 us
 // for 64x64 tiles of the two-stage kernel at four blocks per CU.
 // float32 GEMMs of at least this K take the register-staged kernel's 128x128
-// tiles (three bfloat16 terms per element, two blocks per CU) when those give
-// seven tenths of the CUs one, or the K split of choose() gives every CU 1.8.
-// Measured on one MI355X against the float32 MFMA kernels: 16 x 1024 x 1536,
-// K = 128 62.8 -> 53.9 us, 192 83.8 -> 72.4, 256 107.9 -> 88.9, 512 208.8 ->
-// 154.0; 2048^3 153 -> 114, 4096^3 984 -> 740, 8192 x 2048 x 2048 520 -> 380,
-// 4096 x 128 x 4096 (16 splits) 48.7 -> 43.0, 2304^2 x 6144 (7) 538 -> 403;
-// one tile per CU: 2048^2 x 512 40.9 -> 34.5, 16 x 512^3 43.0 -> 35.1, half a
-// CU's: 2048^2 x 256 (64x64 tiles before) 24.4 -> 22.8.  Shorter K is bound by
-// loads and stores, which two blocks per CU keep fewer of in flight than the
-// direct-load kernel's four (the GDN products, 1024 x 128^3, 52.2 -> 56.4).
+// tiles (three bfloat16 terms per element, eight products, two blocks per CU)
+// when those give seven tenths of the CUs one, or the K split of choose() gives
+// every CU 1.8.
+// Measured on one MI355X against the float32 MFMA kernels: 16 x 1024 x 1536, K
+// = 192 81 -> 76 us, 256 106 -> 97, 512 198 -> 175; 2048^3 158 -> 126, 4096^3
+// 952 -> 864, 8192 x 2048 x 2048 504 -> 432, 4096 x 128 x 4096 (16 splits) 48 ->
+// 44, 2304^2 x 6144 (7) 552 -> 457; one tile per CU: 2048^2 x 512 42.9 -> 39.2,
+// 16 x 512^3 43.7 -> 38.7, half a CU's: 2048^2 x 256 (64x64 tiles before) 25.5 ->
+// 24.0.  Shorter K is bound by loads and stores, which two blocks per CU keep
+// fewer of in flight than the direct-load kernel's four.
 #ifndef PE_GEMM_RS_F32_MIN_K
 #define PE_GEMM_RS_F32_MIN_K 192
 #endif
 // ... and operands that the direct-load kernel cannot take (unaligned rows or
 // bases; element loads otherwise) from this K: 2001 x 3003, K = 75 21.9 ->
-// 17.3 us, 131 31.0 -> 23.7 and (k contiguous) 33.8 -> 22.5.
+// 17.1 us, 131 31.4 -> 23.2 and (k contiguous) 33.6 -> 22.0.
 #ifndef PE_GEMM_RS_F32_MIN_K_ANY
 #define PE_GEMM_RS_F32_MIN_K_ANY 64
 #endif

@@ -10,18 +10,21 @@
 //
 // float32: each element x is split into x0 + x1 + x2, x0 the bfloat16 nearest
 // to x, x1 the one nearest to x - x0, x2 = x - x0 - x1, which 8 bits hold: the
-// split is exact.  A product x y is summed as x0 y0 (one accumulator) and x0
-// y1 + x1 y0 + x1 y1 + x0 y2 + x2 y0 (another), products exact, sums float32;
-// what is left out is below 2^-25 |x y|, under float32's own rounding of the
-// product.  Six v_mfma_f32_32x32x16_bf16 take the place of eight
-// v_mfma_f32_32x32x2_f32 of twice the length: 2.7 times the rate.  The large
-// terms' sums round once per 16 k instead of once per 2 k, so the results are
-// nearer to 64 bits than float32 MFMAs' (relative error at K = 128 / 777 /
-// 4096: 6.5e-8 / 1.6e-7 / 4.0e-7 against 2.0e-7 / 5.0e-7 / 1.1e-6).  The split
-// needs the low term to stay a normal bfloat16 and the sums to stay clear of
-// overflow: elements below 2^-103 in magnitude (zero excepted) and sums of
-// 2^127 and above, inf and NaN among them, mark the tile, and a marked tile
-// is computed again on float32 MFMAs.
+// split is exact, |x1| <= 2^-8 |x|, |x2| <= 2^-17 |x|.  A product x y is summed
+// as x0 y0 (one accumulator) and x0 y1 + x1 y0 + x1 y1 + x0 y2 + x2 y0 + x1 y2
+// + x2 y1 (another), products exact, sums float32; x2 y2, below 2^-33 |x y|, is
+// left out.  A sum with a single non-zero product is that product rounded once
+// but for the low accumulator's own roundings, 2^-28 of it (4 million normal
+// pairs emulated: largest error 5.99e-8, 5.96e-8 rounded once, 0.1 % of values
+// differ; without x1 y2 and x2 y1, up to 2^-24.1 |x y|, 1.0e-7 and 4 %).  Eight
+// v_mfma_f32_32x32x16_bf16 take the place of eight v_mfma_f32_32x32x2_f32 of
+// twice the length: twice the rate.  The large terms' sums round once per 16 k
+// instead of once per 2 k, so longer sums are nearer to 64 bits than float32
+// MFMAs' (relative error at K = 192 / 777 / 4096: 7.8e-8 / 1.6e-7 / 4.0e-7
+// against 2.5e-7 / 5.0e-7 / 1.2e-6).  The split needs the low term to stay a
+// normal bfloat16 and the sums to stay clear of overflow: elements below 2^-103
+// in magnitude (zero excepted) and sums of 2^127 and above, inf and NaN among
+// them, mark the tile, and a marked tile is computed again on float32 MFMAs.
 //
 // Two LDS stages and two register sets per block: during a slab's MFMAs the
 // next slab is converted and stored to the other stage (float32: a third of a
@@ -32,12 +35,13 @@
 // fragment reads of the L_MN operands are DlOperand's for float16, one plane
 // per term; L_K rows are swizzled for the same reads.
 //
-// Measured on one MI355X (cold operands): float16 2001 x 1537 x 3003 209 -> 50
-// us, 3001 x 5003 x 3011 775 -> 190; float32 4096^3 962 -> 731 us (188
-// TFLOP/s), 16 x 1000 x 777 x 1536 278-314 -> 227-233, 2001 x 1537 x 3003 258
-// -> 140.  float32 counters at 4096^3: matrix cores 63 % busy at 1.56 GHz,
-// where the float32 kernel runs 89 % at 2.2: the part is at its power limit,
-// and the conversion's vector work costs clock.  Tried: the compiler's own
+// Measured on one MI355X: float16 2001 x 1537 x 3003 207 -> 47 us (cold 208 ->
+// 43), 3001 x 5003 x 3011 944 -> 185; float32 4096^3 952 -> 864 us (159
+// TFLOP/s), 16 x 1000 x 777 x 1536 cold 277 -> 251, 2001 x 1537 x 3003 257 ->
+// 161; with six products (x1 y2 and x2 y1 left out) 733, 213 and 140.  float32
+// counters at 4096^3, of that form: matrix cores 63 % busy at 1.56 GHz, where
+// the float32 kernel runs 89 % at 2.2: the part is at its power limit, and the
+// conversion's vector work costs clock.  Tried on it: the compiler's own
 // schedule 770 us, no low accumulators (64 registers fewer, no gain, errors as
 // float32's), three blocks per CU (spills), no check of small elements 723.
 #pragma once
@@ -410,6 +414,8 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_rs_kernel(GemmArgs g)
                     mm(1, 1, lo);
                     mm(0, 2, lo);
                     mm(2, 0, lo);
+                    mm(1, 2, lo);
+                    mm(2, 1, lo);
                 } else {
 #pragma unroll
                     for (int i = 0; i < FM; ++i)
@@ -432,7 +438,7 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_rs_kernel(GemmArgs g)
         // Steady state, slab s of parity p: its MFMAs, slab s + 1 to the other
         // stage, the loads of slab s + 3.  float32: the conversion of slab s + 1 runs between the
         // MFMAs of slab s, a third of a pair's split (four or five vector
-        // instructions) after each, so that the matrix core and the vector
+        // instructions) after each of the first 24, so that the matrix core and the vector
         // unit work at the same time whatever the other waves of the SIMD do;
         // the compiler alone runs the two one after the other.
         auto fast = [&](auto p, auto q) {
@@ -462,14 +468,14 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_rs_kernel(GemmArgs g)
                         for (int j = 0; j < FN; ++j) fb[st][e][j] = OB::frag(sb + e * OB::PLANE, lob, wn * WN, j, st);
                     }
                 __builtin_amdgcn_sched_barrier(0);
-                constexpr int NVEC = OA::NV + OB::NV, PIECES = NVEC * 6, SLOTS = 6 * FM * FN * STEPS;
+                constexpr int NVEC = OA::NV + OB::NV, PIECES = NVEC * 6, SLOTS = 8 * FM * FN * STEPS;
                 constexpr int PER = (PIECES + SLOTS - 1) / SLOTS;
-                constexpr int PI[6] = {0, 0, 1, 1, 0, 2}, QI[6] = {0, 1, 0, 1, 2, 0};
+                constexpr int PI[8] = {0, 0, 1, 1, 0, 2, 1, 2}, QI[8] = {0, 1, 0, 1, 2, 0, 2, 1};
                 float ra = 0.0f, rb = 0.0f;
                 uint32_t tt[2][3];
 #pragma unroll
                 for (int slot = 0; slot < SLOTS; ++slot) {
-                    const int st = slot / (6 * FM * FN), pr = slot / (FM * FN) % 6, i = slot / FN % FM, j = slot % FN;
+                    const int st = slot / (8 * FM * FN), pr = slot / (FM * FN) % 8, i = slot / FN % FM, j = slot % FN;
                     f32x16& c = pr == 0 ? acc[i][j] : lo[i][j];
                     c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[st][PI[pr]][i]),
                                                                 __builtin_bit_cast(bf16x8, fb[st][QI[pr]][j]), c, 0, 0, 0);

@@ -27,9 +27,9 @@ def _operands(eq, nb, M, N, K, dtype, seed, off=0):
 
 def _check(eq, a, b, K):
     """Within K roundings of sum |a||b|, the bound of any order of K fused
-    terms (the split's omitted part is below half a rounding per term), each
-    2^-24 of a normal result or 2^-150 of a subnormal one, and the same bits
-    on a second call."""
+    terms, each 2^-24 of a normal result or 2^-150 of a subnormal one, and the
+    same bits on a second call.  (Too wide to see an error in the third term:
+    test_float32_single_products and test_float32_error_at_edges do.)"""
     got = einsum(eq, a, b)
     want = torch.einsum(eq, a.double(), b.double())
     mag = torch.einsum(eq, a.double().abs(), b.double().abs())
@@ -59,6 +59,58 @@ def test_float16_unaligned_rows(eq, nb, M, N, K):
 def test_float32_as_bfloat16_terms(eq, nb, M, N, K, off):
     a, b = _operands(eq, nb, M, N, K, torch.float32, M + N + K, off)
     _check(eq, a, b, K)
+
+
+# Sizes that float32 operands take the kernel at whatever their alignment:
+# tiles without much padding, K tails, tiles that end inside a vector, element
+# offsets, K splits.
+EDGES = [(180, 127, 125, 64, 1), (180, 125, 128, 67, 0), (90, 255, 100, 79, 0), (180, 126, 97, 81, 3),
+         (3, 1025, 1023, 101, 0), (180, 128, 127, 192, 0), (90, 128, 252, 193, 2), (3, 1021, 1026, 207, 0),
+         (1, 1700, 1800, 777, 0), (1, 767, 765, 4099, 1), (1, 768, 768, 4096, 0)]
+
+
+@pytest.mark.parametrize("eq", LAYOUTS)
+@pytest.mark.parametrize("nb,M,N,K,off", EDGES)
+def test_float32_single_products(eq, nb, M, N, K, off):
+    """Sums with one non-zero product are that product rounded once, but for
+    seven roundings of the low accumulator (at most 2^-6.9 of it, so 2^-28.1)
+    and the omitted x2 y2 (2^-33), twice that if sums are cut off: 1 + 2^-3
+    roundings."""
+    a, b = _operands(eq, nb, M, N, K, torch.float32, M + K, off)
+    s1 = eq.split("->")[0].split(",")[1]
+    kn = b if s1 == "bjk" else b.transpose(1, 2)
+    at = (torch.arange(N, device="cuda") * 7 + 3) % K
+    pick = torch.zeros(K, N, device="cuda")
+    pick[at, torch.arange(N, device="cuda")] = 1.0
+    kn.mul_(pick)
+    row = a if eq.startswith("bij") else a.transpose(1, 2)
+    for scale in (1.0,):
+        a.mul_(scale), b.mul_(scale)
+        want = row[:, :, at].double() * kn[:, at, torch.arange(N, device="cuda")].double()[:, None, :]
+        got = einsum(eq, a, b).double()
+        bad = (got - want).abs() > EPS * (1 + 2.0 ** -3) * want.abs() + 2.0 ** -149
+        assert not bool(bad.any()), (scale, int(bad.sum()), float(((got - want) / want).abs().max()))
+
+
+@pytest.mark.parametrize("eq", LAYOUTS)
+@pytest.mark.parametrize("nb,M,N,K,off", EDGES)
+def test_float32_error_at_edges(eq, nb, M, N, K, off):
+    """The relative error against 64 bits is well below that of float32 matrix
+    cores (the explicit 128x128 tile), which round eight times as often; a
+    wrong or missing term, or the other kernel, is above the line."""
+    a, b = _operands(eq, nb, M, N, K, torch.float32, M + N, off)
+    want = torch.einsum(eq, a.double(), b.double())
+    ta, tb = not eq.startswith("bij"), eq.split("->")[0].split(",")[1] == "bkj"
+    d = launch.GemmDesc(dtype=launch.DT_F32, batch_shape=[nb], a_bstride=[M * K], b_bstride=[K * N], c_bstride=[M * N],
+                        M=M, N=N, K=K, a_ms=1 if ta else K, a_ks=M if ta else 1, b_ks=1 if tb else N,
+                        b_ns=K if tb else 1, c_ms=N, c_ns=1, a_numel=nb * M * K, b_numel=nb * K * N,
+                        c_numel=nb * M * N, split_k=1, tile=128)
+    got, ref = einsum(eq, a, b), torch.empty_like(want, dtype=torch.float32)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert abi.bind().pe_gemm(ctypes.byref(abi.gemm_desc(d)), *(ctypes.c_void_p(t.data_ptr()) for t in (a, b, ref)),
+                              None, ctypes.c_int64(0), st) == 0
+    e = [float((x.double() - want).norm() / want.norm()) for x in (got, ref)]
+    assert e[0] <= 0.6 * e[1], e
 
 
 @pytest.mark.parametrize("eq,layout", [(LAYOUTS[0], (0, 1)), (LAYOUTS[1], (0, 0)), (LAYOUTS[2], (1, 1))])
