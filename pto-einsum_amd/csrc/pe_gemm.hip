@@ -95,6 +95,18 @@
 #define PE_GEMM_RS_F32_MIN_K_ANY 64
 #endif
 
+// ... and where 128x128 tiles cover at most this much more than 64x64 ones, for
+// direct-load operands and for others: 100 x 130 x 260 (1.6 times), K = 256, ran
+// 45.6 us against 36.3 on float32 64x64 tiles, 82 x 152 x 400 (1.52), K = 512,
+// 1.01 to 1.10 of their time, 37 x 132 x 1000 (1.33) 1.00 to 1.05, 4 x 1040 x
+// 1040 (1.12), K = 256, 1.04; 60 x 384 x 384 (1.0) 0.81 to 0.85.
+#ifndef PE_GEMM_RS_F32_MAX_PAD
+#define PE_GEMM_RS_F32_MAX_PAD 1.1
+#endif
+#ifndef PE_GEMM_RS_F32_MAX_PAD_ANY
+#define PE_GEMM_RS_F32_MAX_PAD_ANY 1.3
+#endif
+
 #ifndef PE_GEMM_RES
 #define PE_GEMM_RES 1
 #endif
@@ -653,6 +665,10 @@ bool rs_choice(const pe_gemm_desc& d, bool dl, int& al, int& bl, GemmChoice& ch)
             ch.bm = ch.bn = 64;
         return true;
     }
+    // What 128x128 tiles cover against 64x64 ones.
+    auto cover = [&](int t) { return double(ceil_div(d.M, t) * t) * double(ceil_div(d.N, t) * t); };
+    const double pad = cover(128) / cover(64);
+    if (pad > (dl ? PE_GEMM_RS_F32_MAX_PAD : PE_GEMM_RS_F32_MAX_PAD_ANY)) return false;
     const int64_t tiles = ch.nbatch_total * ceil_div(d.M, 128) * ceil_div(d.N, 128), cus = cu_count();
     const bool whole = 10 * tiles >= 7 * cus;
     const bool split = ch.bm == 128 && ch.nsplit > 1 && 10 * tiles * ch.nsplit >= 18 * cus;
@@ -665,7 +681,8 @@ bool rs_choice(const pe_gemm_desc& d, bool dl, int& al, int& bl, GemmChoice& ch)
                (n > 1 ? 100.0 + 3.2e-5 * double(n) * double(ch.nbatch_total) * double(d.M) * double(d.N) : 0.0);
     };
     if (split && (!whole || cost(ch.nsplit, ch.k_per_split) < cost(1, d.K))) return true;
-    if (!whole || (ch.nsplit > 1 && d.K < PE_GEMM_RS_F32_MIN_K)) return false;
+    if (!whole) return false;
+    if (ch.nsplit > 1 && (d.K < PE_GEMM_RS_F32_MIN_K || pad > PE_GEMM_RS_F32_MAX_PAD)) return false;
     ch.bm = ch.bn = 128;
     ch.nsplit = 1;
     ch.k_per_split = int(d.K);

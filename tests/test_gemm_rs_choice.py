@@ -93,3 +93,16 @@ def test_split_does_not_depend_on_alignment(M, N, K, dtype):
         infos.append(([info[2], info[3] if info[2] > 1 else K], int(lib.pe_gemm_workspace_bytes(ctypes.byref(cd)))))
         assert infos[-1][1] >= (infos[-1][0][0] * M * N * 4 if infos[-1][0][0] > 1 else 0)
     assert infos[0] == infos[1]
+
+
+@pytest.mark.parametrize("nb,M,N,K,al,bl,taken", [
+    (100, 130, 260, 256, "k", "n", False), (82, 152, 400, 512, "n", "n", False), (37, 132, 1000, 1024, "k", "k", False),
+    (4, 1040, 1040, 256, "n", "n", False), (60, 384, 384, 256, "n", "n", True), (16, 1000, 1536, 777, "n", "n", True),
+    (100, 130, 260, 257, "k", "n", False), (3, 1025, 1023, 101, "k", "n", True), (90, 129, 255, 65, "n", "k", False),
+])
+def test_float32_padding_rule(nb, M, N, K, al, bl, taken):
+    """Its 128x128 tiles only where they cover little more than 64x64 ones: 1.1
+    times, 1.3 for extents that the direct-load kernel cannot take."""
+    info, ws = _choice(M, N, K, nb=nb, al=al, bl=bl)
+    assert info[2] == 1 and ws == 0
+    assert (info[:2] == [128, 128]) == taken
