@@ -24,7 +24,9 @@
 // against 2.5e-7 / 5.0e-7 / 1.2e-6).  The split needs the low term to stay a
 // normal bfloat16 and the sums to stay clear of overflow: elements below 2^-103
 // in magnitude (zero excepted) and sums of 2^127 and above, inf and NaN among
-// them, mark the tile, and a marked tile is computed again on float32 MFMAs.
+// them, mark the tile, as do sums below 2^-110 in a tile with elements below 2^-60
+// (terms that are subnormal round at 2^-150 each); a marked tile is computed
+// again on float32 MFMAs.
 //
 // Two LDS stages and two register sets per block: during a slab's MFMAs the
 // next slab is converted and stored to the other stage (float32: a third of a
@@ -320,7 +322,7 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_rs_kernel(GemmArgs g)
     constexpr int STAGE = OA::ELEMS + OB::ELEMS;
     static_assert(!kF32 || STAGE * 4 >= BK * (OA::FLD + OB::FLD) * 4, "the float32 pass fits the two stages");
     __shared__ __attribute__((aligned(16))) _Float16 lds[2 * STAGE];
-    __shared__ int redo;
+    __shared__ int redo[3];  // the tile again; it has small elements, small sums
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -512,7 +514,7 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_rs_kernel(GemmArgs g)
         };
         load_part(0, first);
         rs_barrier();  // the last tile's reads are done
-        if (kF32 && tid == 0) redo = 0;
+        if (kF32 && tid < 3) redo[tid] = 0;
         if (steady && nslabs > 1) {
             OA::load_full(na, offa, xa[1]);
             OB::load_full(nb, offb, xb[1]);
@@ -553,9 +555,10 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_rs_kernel(GemmArgs g)
 
         if constexpr (kF32) {
             // 2 |x| - 1 of the smallest element against 2^-103, the largest
-            // sum against 2^127.
-            bool again = low < (24u << 24) - 1u;
-            uint32_t top = 0;
+            // sum against 2^127.  Elements below 2^-60 with sums below 2^-110
+            // (zero among them): terms may be subnormal and round at 2^-150
+            // each, where float32 products round once.
+            uint32_t top = 0, least = 0xffffffffu;
 #pragma unroll
             for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -563,12 +566,15 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_rs_kernel(GemmArgs g)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
                         acc[i][j][r] = acc[i][j][r] + lo[i][j][r];
-                        top = max(top, __builtin_bit_cast(uint32_t, float(acc[i][j][r])) << 1);
+                        const uint32_t m = __builtin_bit_cast(uint32_t, float(acc[i][j][r])) << 1;
+                        top = max(top, m);
+                        least = min(least, m);
                     }
-            again = again || top >= (254u << 24);
-            if (again) redo = 1;
+            if (low < (24u << 24) - 1u || top >= (254u << 24)) redo[0] = 1;
+            if (low < (67u << 24) - 1u) redo[1] = 1;
+            if (least < (17u << 24)) redo[2] = 1;
             rs_barrier();
-            if (redo) {
+            if (redo[0] || (redo[1] && redo[2])) {
                 // The tile again, on float32 MFMAs.
                 float* const fa32 = reinterpret_cast<float*>(lds);
                 float* const fb32 = fa32 + BK * OA::FLD;

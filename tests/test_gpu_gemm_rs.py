@@ -75,7 +75,8 @@ def test_float32_single_products(eq, nb, M, N, K, off):
     """Sums with one non-zero product are that product rounded once, but for
     seven roundings of the low accumulator (at most 2^-6.9 of it, so 2^-28.1)
     and the omitted x2 y2 (2^-33), twice that if sums are cut off: 1 + 2^-3
-    roundings."""
+    roundings.  Scaled operands: products whose terms, or which themselves, are
+    subnormal (tiles that float32 matrix cores compute again)."""
     a, b = _operands(eq, nb, M, N, K, torch.float32, M + K, off)
     s1 = eq.split("->")[0].split(",")[1]
     kn = b if s1 == "bjk" else b.transpose(1, 2)
@@ -84,7 +85,7 @@ def test_float32_single_products(eq, nb, M, N, K, off):
     pick[at, torch.arange(N, device="cuda")] = 1.0
     kn.mul_(pick)
     row = a if eq.startswith("bij") else a.transpose(1, 2)
-    for scale in (1.0,):
+    for scale in (1.0, 2.0 ** -50, 2.0 ** -9, 2.0 ** -7, 2.0 ** -6):    # 2^-50, -59, -66, -72 in all
         a.mul_(scale), b.mul_(scale)
         want = row[:, :, at].double() * kn[:, at, torch.arange(N, device="cuda")].double()[:, None, :]
         got = einsum(eq, a, b).double()
