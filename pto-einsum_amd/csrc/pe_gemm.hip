@@ -79,18 +79,18 @@
 // when those give seven tenths of the CUs one, or the K split of choose() gives
 // every CU 1.8.
 // Measured on one MI355X against the float32 MFMA kernels: 16 x 1024 x 1536, K
-// = 192 81 -> 76 us, 256 106 -> 97, 512 198 -> 175; 2048^3 158 -> 126, 4096^3
-// 952 -> 864, 8192 x 2048 x 2048 504 -> 432, 4096 x 128 x 4096 (16 splits) 48 ->
-// 44, 2304^2 x 6144 (7) 552 -> 457; one tile per CU: 2048^2 x 512 42.9 -> 39.2,
-// 16 x 512^3 43.7 -> 38.7, half a CU's: 2048^2 x 256 (64x64 tiles before) 25.5 ->
-// 24.0.  Shorter K is bound by loads and stores, which two blocks per CU keep
-// fewer of in flight than the direct-load kernel's four.
+// = 192 81 -> 75 us, 256 103 -> 95, 512 195 -> 170; 2048^3 155 -> 126, 4096^3
+// 943 -> 822, 8192 x 2048 x 2048 503 -> 414, 4096 x 128 x 4096 (16 splits) 47.4
+// -> 43.1, 2304^2 x 6144 (7) 543 -> 448; one tile per CU: 2048^2 x 512 43.5 ->
+// 38.6, 16 x 512^3 43.6 -> 38.8, half a CU's: 2048^2 x 256 (64x64 tiles before)
+// 25.2 -> 23.5.  Shorter K is bound by loads and stores, which two blocks per CU
+// keep fewer of in flight than the direct-load kernel's four.
 #ifndef PE_GEMM_RS_F32_MIN_K
 #define PE_GEMM_RS_F32_MIN_K 192
 #endif
 // ... and operands that the direct-load kernel cannot take (unaligned rows or
 // bases; element loads otherwise) from this K: 2001 x 3003, K = 75 21.9 ->
-// 17.1 us, 131 31.4 -> 23.2 and (k contiguous) 33.6 -> 22.0.
+// 17.1 us, 131 30.7 -> 22.5 and (k contiguous) 33.3 -> 21.3.
 #ifndef PE_GEMM_RS_F32_MIN_K_ANY
 #define PE_GEMM_RS_F32_MIN_K_ANY 64
 #endif

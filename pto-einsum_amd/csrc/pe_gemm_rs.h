@@ -21,12 +21,16 @@
 // twice the length: twice the rate.  The large terms' sums round once per 16 k
 // instead of once per 2 k, so longer sums are nearer to 64 bits than float32
 // MFMAs' (relative error at K = 192 / 777 / 4096: 7.8e-8 / 1.6e-7 / 4.0e-7
-// against 2.5e-7 / 5.0e-7 / 1.2e-6).  The split needs the low term to stay a
-// normal bfloat16 and the sums to stay clear of overflow: elements below 2^-103
-// in magnitude (zero excepted) and sums of 2^127 and above, inf and NaN among
-// them, mark the tile, as do sums below 2^-110 in a tile with elements below 2^-60
-// (terms that are subnormal round at 2^-150 each); a marked tile is computed
-// again on float32 MFMAs.
+// against 2.5e-7 / 5.0e-7 / 1.2e-6).
+//
+// Both operands are scaled by 2^24 first, so that every float32, subnormal ones
+// too, splits into normal bfloat16 terms, and the sums by 2^-48 afterwards: terms
+// of products down to 2^-149 stay normal as well.  Scaled sums of 2^127 and above
+// (2^79 unscaled), inf and NaN among them, as elements of 2^104 and above become,
+// mark the tile, and a marked tile is computed again on float32 MFMAs.  (Without
+// the scale, elements below 2^-103 had to mark it: scores under a decay of 0.95
+// a position times values, 4096 x 4096 x 128, 81.7 us, now 39.7; float32 MFMAs
+// 45.9.)
 //
 // Two LDS stages and two register sets per block: during a slab's MFMAs the
 // next slab is converted and stored to the other stage (float32: a third of a
@@ -38,9 +42,9 @@
 // per term; L_K rows are swizzled for the same reads.
 //
 // Measured on one MI355X: float16 2001 x 1537 x 3003 207 -> 47 us (cold 208 ->
-// 43), 3001 x 5003 x 3011 944 -> 185; float32 4096^3 952 -> 864 us (159
-// TFLOP/s), 16 x 1000 x 777 x 1536 cold 277 -> 251, 2001 x 1537 x 3003 257 ->
-// 161; with six products (x1 y2 and x2 y1 left out) 733, 213 and 140.  float32
+// 43), 3001 x 5003 x 3011 944 -> 185; float32 4096^3 943 -> 822 us (167
+// TFLOP/s), 16 x 1000 x 777 x 1536 cold 277 -> 245, 2001 x 1537 x 3003 259 ->
+// 156; with six products (x1 y2 and x2 y1 left out) 733, 217 and 140.  float32
 // counters at 4096^3, of that form: matrix cores 63 % busy at 1.56 GHz, where
 // the float32 kernel runs 89 % at 2.2: the part is at its power limit, and the
 // conversion's vector work costs clock.  Tried on it: the compiler's own
@@ -71,6 +75,11 @@ struct RsVec<F16> {
     typedef _Float16 type __attribute__((ext_vector_type(8)));
     typedef _Float16 utype __attribute__((ext_vector_type(8), aligned(2)));
 };
+
+// Factor of both float32 operands before the split: the last bit of any
+// float32, 2^-149 at the least, becomes 2^-125 or more, so that no term is a
+// subnormal bfloat16.
+constexpr float kRsScale = 0x1p24f;
 
 // Two floats rounded to nearest even, a in the low half.
 __device__ __forceinline__ uint32_t rs_pack(float a, float b) {
@@ -245,9 +254,8 @@ struct RsOperand {
 #pragma unroll
         for (int e = 0; e < 3; ++e) *reinterpret_cast<u32x2*>(p + e * PLANE) = u32x2{tt[0][e], tt[1][e]};
     }
-    // The thread's vectors into LDS; float32: split, `low` keeping the least
-    // 2 |x| - 1 of them (zero wraps to the largest value).
-    __device__ __forceinline__ static void store(_Float16* lds, int tid, const X (&x)[NV], uint32_t& low) {
+    // The thread's vectors into LDS; float32: scaled and split.
+    __device__ __forceinline__ static void store(_Float16* lds, int tid, const X (&x)[NV]) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             int r, k;
@@ -256,11 +264,9 @@ struct RsOperand {
                 *reinterpret_cast<X*>(lds + at(r, k)) = x[v];
             } else {
                 uint32_t tt[2][3];
-                rs_split2(x[v][0], x[v][1], tt[0]);
-                rs_split2(x[v][2], x[v][3], tt[1]);
+                rs_split2(x[v][0] * kRsScale, x[v][1] * kRsScale, tt[0]);
+                rs_split2(x[v][2] * kRsScale, x[v][3] * kRsScale, tt[1]);
                 store_terms(lds, tid, v, tt);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) low = min(low, (__builtin_bit_cast(uint32_t, float(x[v][j])) << 1) - 1u);
             }
         }
     }
@@ -322,7 +328,7 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_rs_kernel(GemmArgs g)
     constexpr int STAGE = OA::ELEMS + OB::ELEMS;
     static_assert(!kF32 || STAGE * 4 >= BK * (OA::FLD + OB::FLD) * 4, "the float32 pass fits the two stages");
     __shared__ __attribute__((aligned(16))) _Float16 lds[2 * STAGE];
-    __shared__ int redo[3];  // the tile again; it has small elements, small sums
+    __shared__ int redo;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -373,7 +379,6 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_rs_kernel(GemmArgs g)
             OA::load_part(A + int64_t(k0) * g.a_ks, g.a_ms, g.a_ks, rows_a, kn, kb + k0, tid, xa[0]);
             OB::load_part(B + int64_t(k0) * g.b_ks, g.b_ns, g.b_ks, rows_b, kn, kb + k0, tid, xb[0]);
         };
-        uint32_t low = 0xffffffffu;
 
         f32x16 acc[FM][FN], lo[kF32 ? FM : 1][kF32 ? FN : 1];
 #pragma unroll
@@ -452,8 +457,8 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_rs_kernel(GemmArgs g)
             }
             if constexpr (!kF32) {
                 multiply(P);
-                OA::store(lds + Q * STAGE, tid, xa[Q], low);
-                OB::store(lds + Q * STAGE + OA::ELEMS, tid, xb[Q], low);
+                OA::store(lds + Q * STAGE, tid, xa[Q]);
+                OB::store(lds + Q * STAGE + OA::ELEMS, tid, xb[Q]);
                 OA::load_full(na, offa, xa[Q]);
                 OB::load_full(nb, offb, xb[Q]);
             } else {
@@ -490,8 +495,8 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_rs_kernel(GemmArgs g)
                             ra = v < OA::NV ? xa[Q][v < OA::NV ? v : 0][2 * half] : xb[Q][v < OA::NV ? 0 : v - OA::NV][2 * half];
                             rb = v < OA::NV ? xa[Q][v < OA::NV ? v : 0][2 * half + 1]
                                             : xb[Q][v < OA::NV ? 0 : v - OA::NV][2 * half + 1];
-                            low = min(low, min((__builtin_bit_cast(uint32_t, ra) << 1) - 1u,
-                                               (__builtin_bit_cast(uint32_t, rb) << 1) - 1u));
+                            ra = ra * kRsScale;
+                            rb = rb * kRsScale;
                         } else {
                             ra = ra - __builtin_bit_cast(float, tt[half][ph - 1] << 16);
                             rb = rb - __builtin_bit_cast(float, tt[half][ph - 1] & 0xffff0000u);
@@ -514,13 +519,13 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_rs_kernel(GemmArgs g)
         };
         load_part(0, first);
         rs_barrier();  // the last tile's reads are done
-        if (kF32 && tid < 3) redo[tid] = 0;
+        if (kF32 && tid == 0) redo = 0;
         if (steady && nslabs > 1) {
             OA::load_full(na, offa, xa[1]);
             OB::load_full(nb, offb, xb[1]);
         }
-        OA::store(lds, tid, xa[0], low);
-        OB::store(lds + OA::ELEMS, tid, xb[0], low);
+        OA::store(lds, tid, xa[0]);
+        OB::store(lds + OA::ELEMS, tid, xb[0]);
         if (steady) {
             if (nslabs > 2) {
                 na += ska;
@@ -548,17 +553,14 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_rs_kernel(GemmArgs g)
             multiply(0);
             if (++s >= nslabs) break;
             rs_barrier();
-            OA::store(lds, tid, xa[0], low);
-            OB::store(lds + OA::ELEMS, tid, xb[0], low);
+            OA::store(lds, tid, xa[0]);
+            OB::store(lds + OA::ELEMS, tid, xb[0]);
             if (!steady && s + 1 < nslabs) load_part(first + s * BK, BK);
         }
 
         if constexpr (kF32) {
-            // 2 |x| - 1 of the smallest element against 2^-103, the largest
-            // sum against 2^127.  Elements below 2^-60 with sums below 2^-110
-            // (zero among them): terms may be subnormal and round at 2^-150
-            // each, where float32 products round once.
-            uint32_t top = 0, least = 0xffffffffu;
+            // The largest scaled sum against 2^127.
+            uint32_t top = 0;
 #pragma unroll
             for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -566,15 +568,12 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_rs_kernel(GemmArgs g)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
                         acc[i][j][r] = acc[i][j][r] + lo[i][j][r];
-                        const uint32_t m = __builtin_bit_cast(uint32_t, float(acc[i][j][r])) << 1;
-                        top = max(top, m);
-                        least = min(least, m);
+                        top = max(top, __builtin_bit_cast(uint32_t, float(acc[i][j][r])) << 1);
+                        acc[i][j][r] = acc[i][j][r] * (1.0f / (kRsScale * kRsScale));
                     }
-            if (low < (24u << 24) - 1u || top >= (254u << 24)) redo[0] = 1;
-            if (low < (67u << 24) - 1u) redo[1] = 1;
-            if (least < (17u << 24)) redo[2] = 1;
+            if (top >= (254u << 24)) redo = 1;
             rs_barrier();
-            if (redo[0] || (redo[1] && redo[2])) {
+            if (redo) {
                 // The tile again, on float32 MFMAs.
                 float* const fa32 = reinterpret_cast<float*>(lds);
                 float* const fb32 = fa32 + BK * OA::FLD;

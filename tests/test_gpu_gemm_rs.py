@@ -159,3 +159,17 @@ def test_float32_range():
     a[6], b[6] = 2.0 ** 60, 1.95 * 2.0 ** 67 / K    # ... and above it
     assert bool(torch.isfinite(einsum(eq, a, b)).all())
     _check(eq, a, b, K)
+
+
+def test_float32_large_elements_and_decays():
+    """Elements that the scale takes past the range against small ones, sums
+    past it that float32 holds, and elements that decay into subnormals."""
+    eq, nb, M, N, K = LAYOUTS[0], 60, 128, 384, 200
+    a, b = _operands(eq, nb, M, N, K, torch.float32, 8)
+    a[2] *= 2.0 ** 110
+    b[2] *= 2.0 ** -100
+    a[5, 3, 7], b[5] = 2.0 ** 127, b[5] * 2.0 ** -20
+    a[8] *= 2.0 ** 40
+    b[8] *= 2.0 ** 45
+    a[11:] *= 2.0 ** -torch.arange(K, device="cuda").float()
+    _check(eq, a, b, K)
