@@ -531,6 +531,7 @@ GemmChoice choose(const pe_gemm_desc& d, bool dl = false, int al = L_MN, int bl 
     }
     int64_t kps = ceil_div(ceil_div(d.K, split), bk) * bk;
     split = std::max<int64_t>(1, ceil_div(d.K, kps));
+    if (!k_ends_fit(d.K)) c.bm = c.bn = 64;  // the one kernel for such K
     c.nsplit = int(split);
     c.k_per_split = int(std::min<int64_t>(kps, INT32_MAX));  // (unsplit K in the last slab below 2^31)
     c.ws_bytes = split > 1 ? split * c.nbatch_total * d.M * d.N * int64_t(sizeof(float)) : 0;
@@ -642,7 +643,7 @@ bool rs_eligible(const pe_gemm_desc& d, int& al, int& bl) {
     al = rs_layout(d.M, d.K, d.a_ms, d.a_ks, vec);
     bl = rs_layout(d.N, d.K, d.b_ns, d.b_ks, vec);
     const int64_t lim = int64_t(1) << 29;  // 32-bit store offsets, as gemm_dl_eligible
-    return d.tile == 0 && d.split_k == 0 && al != L_GENERIC && bl != L_GENERIC &&
+    return d.tile == 0 && d.split_k == 0 && k_ends_fit(d.K) && al != L_GENERIC && bl != L_GENERIC &&
            255 * (d.c_ms + d.c_ns) < lim && 255 * (d.N + 1) < lim;
 }
 

@@ -17,9 +17,9 @@ namespace pe {
 // persist: 0 launches one block per tile; > 0 caps the grid at that many
 // blocks per CU; < 0 caps it at this kernel's own occupancy (every block
 // resident, each walking several tiles).
-template <int BM, int BN, int AL, int BL>
+template <int BM, int BN, int AL, int BL, bool LONGK = false>
 static hipError_t go(const GemmArgs& g, int persist, hipStream_t s) {
-    const auto kernel = gemm_kernel<F32, BM, BN, PE_GEMM_F32_BK, bool(PE_GEMM_F32_KC), PE_GEMM_F32_NBUF, AL, BL>;
+    const auto kernel = gemm_kernel<F32, BM, BN, PE_GEMM_F32_BK, bool(PE_GEMM_F32_KC), PE_GEMM_F32_NBUF, AL, BL, LONGK>;
     GemmArgs a = g;
     if (persist != 0) {
         static const int resident = [&] {
@@ -80,6 +80,8 @@ int gemm_occupancy_f32(int bm, int bn) {
 
 hipError_t launch_gemm_f32(int bm, int bn, int al, int bl, int persist, const GemmArgs& g,
                            hipStream_t s) {
+    // K so near 2^31 that its ranges may end past it: one kernel for all strides.
+    if (!k_ends_fit(g.K)) return go<64, 64, L_GENERIC, L_GENERIC, true>(g, persist, s);
     if (bm == 256) return go_a<256, 128>(al, bl, g, persist, s);
     if (bn == 256) return go_a<128, 256>(al, bl, g, persist, s);
     if (bm == 192) return go_a<192, 128>(al, bl, g, persist, s);

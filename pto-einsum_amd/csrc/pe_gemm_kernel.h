@@ -249,7 +249,8 @@ struct TileWalk {
 #endif
 
 
-template <typename E, int BM, int BN, int BK, bool KC, int NBUF, int ALAYOUT, int BLAYOUT>
+// LONGK: for K whose ranges or slabs may end past 2^31 (k_ends_fit).
+template <typename E, int BM, int BN, int BK, bool KC, int NBUF, int ALAYOUT, int BLAYOUT, bool LONGK = false>
 __global__ __launch_bounds__(kGemmThreads, 2) void gemm_kernel(GemmArgs g) {
     using G = GemmGeom<E, BM, BN, BK, KC, NBUF>;
     using T = typename E::T;
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_kernel(GemmArgs g) {
         x.m0 = tm * BM;
         x.n0 = tn * BN;
         const int kb = int(x.split) * g.k_per_split;
-        x.k_len = k_range(g.K, kb, g.k_per_split);
+        x.k_len = LONGK ? k_range(g.K, kb, g.k_per_split) : min(g.K, kb + g.k_per_split) - kb;
         x.rows_a = g.M - x.m0;
         x.rows_b = g.N - x.n0;
         x.A = static_cast<const T*>(g.a) + a_off + int64_t(x.m0) * g.a_ms + int64_t(kb) * g.a_ks;
@@ -326,7 +327,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_kernel(GemmArgs g) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-        const int nslabs = k_slabs(cur_t.k_len, BK);
+        const int nslabs = LONGK ? k_slabs(cur_t.k_len, BK) : (cur_t.k_len + BK - 1) / BK;
         int k_left = cur_t.k_len;
         la.store(lds_a[0], tid);
         lb.store(lds_b[0], tid);

@@ -359,8 +359,8 @@ __global__ __launch_bounds__(kGemmThreads, MINB) void gemm_rs_kernel(GemmArgs g)
         const int backm = OA::back(g.M - tm * BM, tm), backn = OB::back(g.N - tn * BN, tn);
         const int m0 = tm * BM - backm, n0 = tn * BN - backn;
         const int kb = int(split) * g.k_per_split;
-        const int k_len = k_range(g.K, kb, g.k_per_split);
-        const int nslabs = k_slabs(k_len, BK);
+        const int k_len = min(g.K, kb + g.k_per_split) - kb;
+        const int nslabs = (k_len + BK - 1) / BK;
         const int rows_a = g.M - m0, rows_b = g.N - n0;
         const T* const A = static_cast<const T*>(g.a) + a_off + int64_t(m0) * g.a_ms + int64_t(kb) * g.a_ks;
         const T* const B = static_cast<const T*>(g.b) + b_off + int64_t(n0) * g.b_ns + int64_t(kb) * g.b_ks;

@@ -22,10 +22,10 @@ constexpr int32_t k_slabs(int32_t len, int32_t bk) {
 }
 
 // Whether every range of K and every slab of it ends below 2^31, however K is
-// split (splits of whole slabs end less than 2^20 past K).  Kernels that form
-// these ends as plain sums take such K only (gemm_dl_eligible): with k_range
-// instead, the direct-load float32 64x64 tiles ran up to 9 % longer (82 x 152 x
-// 400, K = 1024, 129 -> 141 us).
+// split (splits of whole slabs end less than 2^20 past K).  GEMM kernels form
+// these ends as plain sums and take such K only, but for one that takes the
+// rest: with k_range in all of them, the direct-load float32 64x64 tiles ran up
+// to 9 % longer (82 x 152 x 400, K = 1024, 129 -> 141 us), staged ones up to 6.
 constexpr bool k_ends_fit(int64_t K) { return K <= INT32_MAX - (1 << 20); }
 
 // Rows (or columns) of a GEMM that run in one launch, the rest in another:
