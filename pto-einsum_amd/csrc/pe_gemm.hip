@@ -883,11 +883,6 @@ extern "C" int pe_gemm(const pe_gemm_desc* d, const void* a, const void* b, floa
         if (v.ws_bytes > 0 && (!ws || ws_bytes < v.ws_bytes))
             return fail(PE_ERR_WORKSPACE, "gemm: split-K workspace missing or too small");
         PE_CHECK_HIP(launch_gemv(*d, v, nb, a, b, c, ws, s));
-        if (v.split > 1 && v.split <= kWaveReduceSplits) {
-            r.nsplit = v.split;
-            r.partial = static_cast<const float*>(ws);
-            PE_CHECK_HIP(launch_splitk_reduce(r, s));
-        }
         return PE_OK;
     }
 

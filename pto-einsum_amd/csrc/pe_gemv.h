@@ -32,8 +32,7 @@ struct GemvPlan {
     int64_t N, blocks, ws_bytes;
 };
 
-// Up to this many splits the caller sums the partials (launch_splitk_reduce,
-// a thread per output); more splits launch_gemv sums itself, a wave per row.
+// Up to this many splits a thread per output sums the partials, more a wave.
 constexpr int kWaveReduceSplits = 16;
 
 GemvPlan gemv_plan(const pe_gemm_desc& d, int64_t nb);

@@ -18,20 +18,29 @@
 //     every KR-th k of its block's range, U loads in flight; the KR partial
 //     sums meet in LDS and are added in order.
 //
-// Few outputs and a long K: K is split over blocks and the partials summed
-// in split order by the GEMM's reduction kernel.  Rows may start at any
-// element (16-byte loads at element alignment where the strides are not
+// Few outputs and a long K: K is split over blocks and the partials are summed
+// in split order or by a wave for each output, in 64 bits.  Rows may start at
+// any element (16-byte loads at element alignment where the strides are not
 // whole vectors); the last K % V elements of a row are read one by one and
 // rows past the end are clamped in bounds and never stored.
 //
+// Sums: a lane or thread adds at most K / LPR or K / KR products in float32,
+// and what could round more often than the matrix cores (they round a block of
+// products once) is added in 64 bits: short rows and columns, the sums of
+// float16 lanes and of a column's threads, the partials.  Over 340 shapes, K =
+// 8 to 2^22, the relative error against 64 bits is 0.01 to 0.93 of the tiles'
+// (sums all in 32 bits but for the float16 lanes': up to 1.14).
+//
 // Measured on one MI355X (W rotated over 1 GiB), GEMM kernels before -> now:
-// f32 8192 x 4096 matvec 46.7 -> 23.1 us (5.8 TB/s; a copy reaches 6.5), the
-// f16 scores and values of 512 heads x 2048 positions x 128 together 165 -> 92
-// us.  Against these shapes: W through ordinary loads 24-31 and 50 + 55 us;
-// four rows per lane for long rows (x shared) 30 us, two 23.6; U = 2 or 8 24.4;
-// eight k in flight per thread for the columns 49, sixteen 60 us (four: 46);
-// 64-bit lane sums exchanged through LDS instead of DPP 66 us for the scores
-// (46), pairwise sums within a lane's vector 55-58 (96 registers either way).
+// f32 8192 x 4096 matvec 46.5 -> 22.1 us (6.1 TB/s; a copy reaches 6.5), the
+// f16 scores and values of 512 heads x 2048 positions x 128 together 152 -> 87
+// us.  W in the Infinity Cache (the same call again): f32 4096^2 ij,j->i 27.9 ->
+// 10.0 us, i,ij->j 28.9 -> 18.7.  Against the first shapes: W through ordinary
+// loads 24-31 and 50 + 55 us; four rows per lane for long rows (x
+// shared) 30 us, two 23.6; U = 2 or 8 24.4; eight k in flight per thread for the
+// columns 49, sixteen 60 us (four: 46); 64-bit lane sums exchanged through LDS
+// instead of DPP 66 us for the scores (46), pairwise sums within a lane's vector
+// 55-58, all products in 64 bits 51.6 for the scores, 54 for the values.
 #include "pe_gemv.h"
 
 #include <algorithm>
@@ -84,7 +93,8 @@ __device__ __forceinline__ float dot4(const typename E::T (&w)[4], const typenam
 // acc + w x, one rounding (in 64 bits float16's product is exact in 32).
 template <typename E, typename A>
 __device__ __forceinline__ A mad(typename E::T w, typename E::T x, A acc) {
-    if constexpr (sizeof(A) == 8) return acc + A(E::to_f32(w) * E::to_f32(x));
+    if constexpr (sizeof(A) == 8 && E::kBytes == 4) return __builtin_fma(double(w), double(x), acc);
+    else if constexpr (sizeof(A) == 8) return acc + A(E::to_f32(w) * E::to_f32(x));
     else return __builtin_fmaf(E::to_f32(w), E::to_f32(x), acc);
 }
 
@@ -96,11 +106,11 @@ __device__ __forceinline__ A dot16(typename Vec16<E>::type w, typename Vec16<E>:
     return acc;
 }
 
-// Type in which the lanes' (and the column kernel's thread rows') partial sums
-// meet: float16 operands in 64 bits, one rounding for all of them.  The matrix
-// cores round a block of products once, which chains and meets in 32 bits do
-// not reach (relative error over K = 64: tiles 5.7e-8, 32 bits 6.6e-8, this
-// 5.2e-8; the times are the same).
+// Type in which the row kernel's lanes' partial sums meet: float16 operands in
+// 64 bits, one rounding for all of them.  The matrix cores round a block of
+// products once, which chains and meets in 32 bits do not reach (relative error
+// over K = 64: tiles 5.7e-8, 32 bits 6.6e-8, this 5.2e-8; the times are the
+// same).
 template <typename E>
 struct Meet {
     using T = float;
@@ -191,9 +201,9 @@ __global__ __launch_bounds__(kThreads) void gemv_row_kernel(GemvArgs g) {
         }
     }
 
-    // Rows of four vectors: all in 64 bits (K = 32: 4.4e-8 through the tiles,
-    // 5.3e-8 with a 32-bit chain).
-    using A = std::conditional_t<LPR == 4, typename Meet<E>::T, float>;
+    // float16 rows of up to eight vectors: all in 64 bits (K = 32: 4.4e-8
+    // through the tiles, 5.3e-8 with a 32-bit chain; K = 33 4.9e-8 and 5.3e-8).
+    using A = std::conditional_t<(LPR <= 8), typename Meet<E>::T, float>;
     A acc[R][U];
 #pragma unroll
     for (int i = 0; i < R; ++i)
@@ -259,27 +269,23 @@ __global__ __launch_bounds__(kThreads) void gemv_row_kernel(GemvArgs g) {
         }
         held += up ? half : 0;
     }
-    constexpr int kLeft = R > LPR ? R / LPR : 1;  // rows a lane still holds
+    static_assert(R <= LPR, "a lane is left with one row");
 #pragma unroll
     for (; m >= 1; m /= 2) s[0] = s[0] + xor_lane(s[0], m);
-    // Lanes that hold the same rows: the first stores.
-    constexpr int kDup = LPR > R ? LPR / R : 1;
-    if (l % kDup != 0) return;
-#pragma unroll
-    for (int i = 0; i < kLeft; ++i) {
-        const uint32_t r = row0 + uint32_t(held + i) * G + grp;
-        if (r >= nrows) continue;
-        if (g.nsplit > 1) {
-            g.partial[int64_t(blockIdx.y) * g.rows + (XROW ? r : batch * uint32_t(g.N) + r)] = float(s[i]);
-        } else if constexpr (XROW) {
-            uint32_t b, n;
-            g.n_div.divmod(r, b, n);
-            int64_t wo, xo, o;
-            batch_offsets(g, b, wo, xo, o);
-            g.out[o + int64_t(n) * g.o_ns] = float(s[i]);
-        } else {
-            g.out[oo + int64_t(r) * g.o_ns] = float(s[i]);
-        }
+    // LPR / R lanes hold the same row: the first stores.
+    if (l % (LPR / R) != 0) return;
+    const uint32_t r = row0 + uint32_t(held) * G + grp;
+    if (r >= nrows) return;
+    if (g.nsplit > 1) {
+        g.partial[int64_t(blockIdx.y) * g.rows + (XROW ? r : batch * uint32_t(g.N) + r)] = float(s[0]);
+    } else if constexpr (XROW) {
+        uint32_t b, n;
+        g.n_div.divmod(r, b, n);
+        int64_t wo, xo, o;
+        batch_offsets(g, b, wo, xo, o);
+        g.out[o + int64_t(n) * g.o_ns] = float(s[0]);
+    } else {
+        g.out[oo + int64_t(r) * g.o_ns] = float(s[0]);
     }
 }
 
@@ -290,7 +296,7 @@ __global__ __launch_bounds__(kThreads) void gemv_col_kernel(GemvArgs g) {
     using X = typename Vec16<E>::type;
     constexpr int V = Vec16<E>::V;
     constexpr int KR = kThreads / CL;
-    __shared__ float red[KR > 1 ? KR * CL * V : 1];
+    __shared__ double red[KR * CL * V];
     const int col = threadIdx.x % CL, kr = threadIdx.x / CL;
     const uint32_t batch = blockIdx.x / g.tiles;
     const int tile = int(blockIdx.x - batch * g.tiles);
@@ -306,76 +312,95 @@ __global__ __launch_bounds__(kThreads) void gemv_col_kernel(GemvArgs g) {
     const T* w = static_cast<const T*>(g.w) + wo + n0;
     const T* x = static_cast<const T*>(g.x) + xo;
 
-    float acc[V];
+    double tot[V];
 #pragma unroll
-    for (int e = 0; e < V; ++e) acc[e] = 0.0f;
+    for (int e = 0; e < V; ++e) tot[e] = 0.0;
     uint32_t k = kb + kr;
-    for (; k + (U - 1) * KR < ke; k += U * KR) {
-        X wv[U];
-        T xv[U];
+    // U k at a time, in float32 or in 64 bits.
+    auto walk = [&](auto zero) {
+        using A = decltype(zero);
+        A acc[V];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            wv[u] = ldw<E, UNAL>(w + int64_t(k + u * KR) * g.w_ks);
-            xv[u] = x[int64_t(k + u * KR) * g.x_ks];
+        for (int e = 0; e < V; ++e) acc[e] = zero;
+        for (; k + (U - 1) * KR < ke; k += U * KR) {
+            X wv[U];
+            T xv[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                wv[u] = ldw<E, UNAL>(w + int64_t(k + u * KR) * g.w_ks);
+                xv[u] = x[int64_t(k + u * KR) * g.x_ks];
+            }
+            if constexpr (V == 8 && U == 4 && sizeof(A) == 4) {
+#pragma unroll
+                for (int e = 0; e < V; ++e) acc[e] = acc[e] + dot4<E>({wv[0][e], wv[1][e], wv[2][e], wv[3][e]}, xv);
+            } else {
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int e = 0; e < V; ++e) acc[e] = mad<E, A>(wv[u][e], xv[u], acc[e]);
+            }
         }
-        if constexpr (V == 8 && U == 4) {
 #pragma unroll
-            for (int e = 0; e < V; ++e) acc[e] = acc[e] + dot4<E>({wv[0][e], wv[1][e], wv[2][e], wv[3][e]}, xv);
-        } else {
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int e = 0; e < V; ++e) acc[e] = __builtin_fmaf(E::to_f32(wv[u][e]), E::to_f32(xv[u]), acc[e]);
-        }
-    }
+        for (int e = 0; e < V; ++e) tot[e] = acc[e];
+    };
+    // 64 bits for a thread's last k, for all of a short K's (float16: sixteen a
+    // thread) and where the thread rows' sums meet: in 32 bits, K = 8 to 64
+    // came out up to 1.14 times as far from 64 bits as through the tiles.
+    if (E::kBytes == 2 && ke - kb <= 16 * KR) walk(0.0);
+    else walk(0.0f);
     for (; k < ke; k += KR) {
         const X wv = ldw<E, UNAL>(w + int64_t(k) * g.w_ks);
-        const float xv = E::to_f32(x[int64_t(k) * g.x_ks]);
+        const T xv = x[int64_t(k) * g.x_ks];
 #pragma unroll
-        for (int e = 0; e < V; ++e) acc[e] = __builtin_fmaf(E::to_f32(wv[e]), xv, acc[e]);
+        for (int e = 0; e < V; ++e) tot[e] = mad<E, double>(wv[e], xv, tot[e]);
     }
     float* out = g.nsplit > 1 ? g.partial + int64_t(blockIdx.y) * g.rows + int64_t(batch) * g.N : g.out + oo;
     const int64_t o_ns = g.nsplit > 1 ? 1 : g.o_ns;
-    if constexpr (KR == 1) {
-        if (n_own < g.N) {
+    // [kr][e][col]: each store and read is a run of CL lanes.
 #pragma unroll
-            for (int e = 0; e < V; ++e)
-                if (n0 + e >= n_own) out[int64_t(n0 + e) * o_ns] = acc[e];
-        }
-    } else {
-        // [kr][e][col]: each store and read is a run of CL lanes.
+    for (int e = 0; e < V; ++e) red[(kr * V + e) * CL + col] = tot[e];
+    __syncthreads();
+    for (int i = threadIdx.x; i < CL * V; i += kThreads) {
+        const int c = i % CL, e = i / CL;
+        double s = red[e * CL + c];
 #pragma unroll
-        for (int e = 0; e < V; ++e) red[(kr * V + e) * CL + col] = acc[e];
-        __syncthreads();
-        for (int i = threadIdx.x; i < CL * V; i += kThreads) {
-            const int c = i % CL, e = i / CL;
-            typename Meet<E>::T s = red[e * CL + c];
-#pragma unroll
-            for (int r = 1; r < KR; ++r) s = s + red[(r * V + e) * CL + c];
-            const int own = (tile * CL + c) * V;
-            const int n = min(own, g.N - V) + e;
-            if (own < g.N && n >= own) out[int64_t(n) * o_ns] = float(s);
-        }
+        for (int r = 1; r < KR; ++r) s = s + red[(r * V + e) * CL + c];
+        const int own = (tile * CL + c) * V;
+        const int n = min(own, g.N - V) + e;
+        if (own < g.N && n >= own) out[int64_t(n) * o_ns] = float(s);
     }
 }
 
-// out[row] = sum of the row's nsplit partials, one wave per row: lane l adds
-// splits l, l + 64, ... in order, then a butterfly (many splits of few rows,
-// where one thread per output would wait for its loads in turn).
+// out[row] = sum of the row's nsplit partials in 64 bits.  WAVE: one wave per
+// row, lane l adding splits l, l + 64, ... in order, then a butterfly (many
+// splits of few rows, where one thread per output would wait for its loads in
+// turn); else a thread per row, in split order.
+template <bool WAVE>
 __global__ __launch_bounds__(kThreads) void gemv_reduce_kernel(GemvArgs g) {
-    const uint32_t row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const uint32_t row = WAVE ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x * kThreads + threadIdx.x;
     if (row >= g.rows) return;
-    const int lane = threadIdx.x & 63;
-    float s = 0.0f;
-    for (int i = lane; i < g.nsplit; i += 64) s = s + g.partial[int64_t(i) * g.rows + row];
+    const int lane = WAVE ? threadIdx.x & 63 : 0;
+    double s = 0.0;
+    if constexpr (WAVE) {
+        for (int i = lane; i < g.nsplit; i += 64) s = s + double(g.partial[int64_t(i) * g.rows + row]);
 #pragma unroll
-    for (int m = 32; m >= 1; m /= 2) s = s + __shfl_xor(s, m);
+        for (int m = 32; m >= 1; m /= 2) s = s + __shfl_xor(s, m);
+    } else {
+        constexpr int U = 8;
+        for (int i = 0; i < g.nsplit; i += U) {
+            float x[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) x[u] = g.partial[int64_t(min(i + u, g.nsplit - 1)) * g.rows + row];
+#pragma unroll
+            for (int u = 0; u < U; ++u) s = s + (i + u < g.nsplit ? double(x[u]) : 0.0);
+        }
+    }
     if (lane == 0) {
         uint32_t b, n;
         g.n_div.divmod(row, b, n);
         int64_t wo, xo, o;
         batch_offsets(g, b, wo, xo, o);
-        g.out[o + int64_t(n) * g.o_ns] = s;
+        g.out[o + int64_t(n) * g.o_ns] = float(s);
     }
 }
 
@@ -509,9 +534,11 @@ hipError_t launch_gemv(const pe_gemm_desc& d, const GemvPlan& p, int64_t nb, con
     void* args[] = {&g};
     hipError_t e = hipLaunchKernel(reinterpret_cast<const void*>(fn), dim3(uint32_t(p.blocks), uint32_t(p.split)),
                                    dim3(kThreads), args, 0, s);
-    if (e != hipSuccess || p.split <= kWaveReduceSplits) return e;
-    return hipLaunchKernel(reinterpret_cast<const void*>(&gemv_reduce_kernel), dim3(uint32_t(ceil_div(g.rows, 4))),
-                           dim3(kThreads), args, 0, s);
+    if (e != hipSuccess || p.split == 1) return e;
+    const bool wave = p.split > kWaveReduceSplits;
+    return hipLaunchKernel(wave ? reinterpret_cast<const void*>(&gemv_reduce_kernel<true>)
+                                : reinterpret_cast<const void*>(&gemv_reduce_kernel<false>),
+                           dim3(uint32_t(ceil_div(g.rows, wave ? 4 : kThreads))), dim3(kThreads), args, 0, s);
 }
 
 }  // namespace pe
