@@ -99,7 +99,8 @@ __device__ __forceinline__ void rs_split2(float a, float b, uint32_t (&t)[3]) {
     }
 }
 
-// One operand's share of a slab of BK k: ROWS rows (m or n).
+// One operand's share of a slab of BK k: ROWS rows (m or n).  (The loads are
+// host functions too: a test runs them against the ends of an operand.)
 template <typename E, int ROWS, int LAYOUT, int BK>
 struct RsOperand {
     using R = RsVec<E>;
@@ -114,7 +115,7 @@ struct RsOperand {
     static_assert(NV >= 1 && kGemmThreads % VPR == 0, "whole vectors per thread");
     static constexpr int FLD = ROWS + 4;                     // float32 pass: LDS pitch of a k row
 
-    __device__ __forceinline__ static void pos(int tid, int v, int& r, int& k) {
+    __host__ __device__ __forceinline__ static void pos(int tid, int v, int& r, int& k) {
         const int a = tid / VPR + v * STEP, c = (tid % VPR) * V;
         r = LAYOUT == L_K ? a : c;
         k = LAYOUT == L_K ? c : a;
@@ -123,7 +124,8 @@ struct RsOperand {
     // slab whose every k is in range.  Rows past the operand repeat its last
     // row (L_K) or last vector (L_MN): they feed outputs that are never
     // stored.
-    __device__ __forceinline__ static void offsets(int64_t rs, int64_t ks, int rows_left, int tid, uint32_t (&o)[NV]) {
+    __host__ __device__ __forceinline__ static void offsets(int64_t rs, int64_t ks, int rows_left, int tid,
+                                                            uint32_t (&o)[NV]) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             int r, k;
@@ -135,24 +137,26 @@ struct RsOperand {
     // L_MN rows that end inside a vector: the tile that would pass them
     // starts `back` rows earlier, so that it ends with them (tiles of
     // operands shorter than a tile keep their place and take load_part).
-    __device__ __forceinline__ static int back(int rows_left, int first_row) {
+    __host__ __device__ __forceinline__ static int back(int rows_left, int first_row) {
         return LAYOUT == L_MN && rows_left < ROWS && rows_left % V != 0 && first_row > 0 ? ROWS - rows_left : 0;
     }
     // Whether offsets() serves a tile: no vector straddles the last row.
-    __device__ __forceinline__ static bool whole(int rows_left) {
+    __host__ __device__ __forceinline__ static bool whole(int rows_left) {
         return LAYOUT == L_K || rows_left >= ROWS || rows_left % V == 0;
     }
-    __device__ __forceinline__ static X vload(const T* p) { return *reinterpret_cast<const typename R::utype*>(p); }
+    __host__ __device__ __forceinline__ static X vload(const T* p) {
+        return *reinterpret_cast<const typename R::utype*>(p);
+    }
 
-    __device__ __forceinline__ static X load_one(const T* base, uint32_t o) {
+    __host__ __device__ __forceinline__ static X load_one(const T* base, uint32_t o) {
         return vload(reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + o));
     }
-    __device__ __forceinline__ static void load_full(const T* base, const uint32_t (&o)[NV], X (&x)[NV]) {
+    __host__ __device__ __forceinline__ static void load_full(const T* base, const uint32_t (&o)[NV], X (&x)[NV]) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) x[v] = load_one(base, o[v]);
     }
     // x moved down by d elements, zeros shifted in (d >= V: all zero).
-    __device__ __forceinline__ static void shift(X& x, int d) {
+    __host__ __device__ __forceinline__ static void shift(X& x, int d) {
         u32x4 w = __builtin_bit_cast(u32x4, x);
         constexpr int E4 = V / 4;  // elements per dword
         if (d >= V) w = u32x4{0, 0, 0, 0};
@@ -166,7 +170,7 @@ struct RsOperand {
         x = __builtin_bit_cast(X, w);
     }
     // Elements n and up of x zeroed (0 <= n).
-    __device__ __forceinline__ static void keep(X& x, int n) {
+    __host__ __device__ __forceinline__ static void keep(X& x, int n) {
 #pragma unroll
         for (int j = 0; j < V; ++j) x[j] = j < n ? x[j] : T(0);
     }
@@ -178,8 +182,8 @@ struct RsOperand {
     // slab is cleared.  k past the end is zero, rows past it are in-bounds
     // values (or zeros) that feed outputs which are never stored.  Every load
     // lies within V elements that the operand has along its contiguous axis.
-    __device__ __forceinline__ static void load_part(const T* base, int64_t rs, int64_t ks, int rows_left, int k_left,
-                                                     int before, int tid, X (&x)[NV]) {
+    __host__ __device__ __forceinline__ static void load_part(const T* base, int64_t rs, int64_t ks, int rows_left,
+                                                              int k_left, int before, int tid, X (&x)[NV]) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             int r, k;
