@@ -50,23 +50,19 @@ def test_float16_unaligned_rows(eq, nb, M, N, K):
     _check(eq, a, b, K)
 
 
-@pytest.mark.parametrize("eq", LAYOUTS)
-@pytest.mark.parametrize("nb,M,N,K,off", [
-    (48, 129, 131, 64, 1), (48, 130, 140, 65, 0), (48, 255, 100, 79, 0), (48, 129, 257, 81, 0), (50, 200, 136, 191, 3),
-    (48, 128, 256, 192, 0), (48, 132, 252, 193, 0), (47, 133, 255, 207, 2), (1, 1700, 1800, 777, 0),
-    (1, 768, 768, 4096, 0), (1, 767, 765, 4099, 0),    # K splits
-])
-def test_float32_as_bfloat16_terms(eq, nb, M, N, K, off):
-    a, b = _operands(eq, nb, M, N, K, torch.float32, M + N + K, off)
-    _check(eq, a, b, K)
-
-
 # Sizes that float32 operands take the kernel at whatever their alignment:
 # tiles without much padding, K tails, tiles that end inside a vector, element
 # offsets, K splits.
 EDGES = [(180, 127, 125, 64, 1), (180, 125, 128, 67, 0), (90, 255, 100, 79, 0), (180, 126, 97, 81, 3),
          (3, 1025, 1023, 101, 0), (180, 128, 127, 192, 0), (90, 128, 252, 193, 2), (3, 1021, 1026, 207, 0),
          (1, 1700, 1800, 777, 0), (1, 767, 765, 4099, 1), (1, 768, 768, 4096, 0)]
+
+
+@pytest.mark.parametrize("eq", LAYOUTS)
+@pytest.mark.parametrize("nb,M,N,K,off", EDGES)
+def test_float32_as_bfloat16_terms(eq, nb, M, N, K, off):
+    a, b = _operands(eq, nb, M, N, K, torch.float32, M + N + K, off)
+    _check(eq, a, b, K)
 
 
 @pytest.mark.parametrize("eq", LAYOUTS)
@@ -138,9 +134,9 @@ def test_float32_range():
     """Elements and sums outside the split's range: inf and NaN reach exactly
     the outputs whose sums hold them, tiny and subnormal elements keep their
     float32 accuracy, sums near the largest float32 stay finite."""
-    eq, nb, M, N, K = LAYOUTS[0], 48, 130, 260, 200
+    eq, nb, M, N, K = LAYOUTS[0], 60, 127, 383, 200
     a, b = _operands(eq, nb, M, N, K, torch.float32, 5)
-    a[3, 7, 11], b[9, 100, 20], a[20, 129, 199] = float("inf"), float("nan"), float("-inf")
+    a[3, 7, 11], b[9, 100, 20], a[20, 126, 199] = float("inf"), float("nan"), float("-inf")
     a[30, 5] = 2.0 ** 120
     b[30, :, 6] = 2.0 ** 9     # overflows to inf as float32 does
     got, want = einsum(eq, a, b), torch.einsum(eq, a.double(), b.double())
