@@ -217,7 +217,7 @@ class EinsumBuilder:
             # A workspace that no kernel touches may be anyone's.
             key = (idx, stream, thread()) if uses_ws else (idx, 0, 0)
             ws = self._workspaces.get(key)
-            if ws is None or (uses_ws and capturing()):
+            if ws is None or (stream and uses_ws and capturing()):    # (the default stream, 0, is never captured)
                 ws = self._workspace(key, dev)
             rc = exec_fn(inp0.data_ptr(), inp1.data_ptr(), out.data_ptr(), ws.data_ptr(), stream)
             if rc:
