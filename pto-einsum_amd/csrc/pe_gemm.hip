@@ -659,9 +659,10 @@ bool rs_choice(const pe_gemm_desc& d, bool dl, int& al, int& bl, GemmChoice& ch)
         return false;
     ch = choose(d);
     if (d.dtype == PE_F16) {
-        // A handful of 128x128 tiles: 64x64 ones (300 x 200 x 100 16.7 -> 6.8
-        // us; from one tile in eight CUs the larger win, 501 x 537 x 503 15.3
-        // against 19.8).
+        // A handful of 128x128 tiles: 64x64 ones (300 x 200 x 100 15.9 us
+        // through element loads, 4.0; from one tile in eight CUs the larger
+        // won, 501 x 537 x 503 15.3 against 19.8, when 64x64 tiles still took
+        // their fragment offsets from an array).
         if (16 * ch.nbatch_total * ceil_div(d.M, 128) * ceil_div(d.N, 128) * ch.nsplit <= cu_count())
             ch.bm = ch.bn = 64;
         return true;
